@@ -334,6 +334,10 @@ static hipError_t gemv_engines(const GemvArgs* ap, hipStream_t st) {
         dim3 block;
         const hipError_t e3 = s2p_gemv_plan_check(&a3);
         if (e3 != hipSuccess) return e3;
+        if (a.M <= 16) { /* loads in the operand layout, every load in flight (gemvr.hip) */
+            const hipError_t er = s2p_gvr_launch(&a, st);
+            if (er != hipErrorNotSupported) return er;
+        }
         const hipError_t pe3 = s2p_gemv3_plan(&a3, &grid, &block, &lds);
         if (pe3 == hipSuccess) {
             switch (a3.wfmt) {
@@ -380,7 +384,9 @@ extern "C" hipError_t s2p_gemv_launch(const GemvArgs* ap, hipStream_t st) {
         if (e4 != hipErrorNotSupported) return e4;
     }
     const hipError_t e = gemv_engines(ap, st);
-    if (e != hipSuccess || !ap->inv_out || ap->epi != GEMV_EPI_RESID || !ap->ssq_out) return e;
+    /* the inverse RMS is read by k_gemm4 only, whose rows are the same M */
+    if (e != hipSuccess || ap->M <= 16 || !ap->inv_out || ap->epi != GEMV_EPI_RESID || !ap->ssq_out)
+        return e;
     return s2p_g4_rms_launch(ap->ssq_out, (ap->N + 15) / 16, ap->M, ap->N, ap->inv_eps,
                              ap->inv_out, st);
 }

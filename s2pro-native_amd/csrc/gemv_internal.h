@@ -63,6 +63,8 @@ typedef struct {
 hipError_t s2p_gemv_launch(const GemvArgs* a, hipStream_t st);
 /* INT4, 16 < M <= 96 (gemm4.hip); hipErrorNotSupported outside that range */
 hipError_t s2p_gemm4_launch(const GemvArgs* a, hipStream_t st);
+/* M <= 16 (gemvr.hip); hipErrorNotSupported outside its shapes */
+hipError_t s2p_gvr_launch(const GemvArgs* a, hipStream_t st);
 /* inv[m] = the rule's inverse RMS of row m < M from per-16-column sums of
  * squares ssq [blocks][GEMV_MAX_M] of rows of K values (gemm4.hip) */
 hipError_t s2p_g4_rms_launch(const float* ssq, int blocks, int M, int K, float eps, float* inv,

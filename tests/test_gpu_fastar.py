@@ -271,3 +271,32 @@ def test_argmax_ties_nan(lib):
         want = int(np.flatnonzero(v == v.max())[0])
         assert got[i] == want, f"row {i}: {got[i]} vs {want}"
     assert got[1] == 7 and got[2] == 0 and got[3] == 11 and got[4] == 2049 and got[5] == 4095
+
+
+def test_frame_rows_past_eight(lib, decoder):
+    """A frame's first-step logits do not depend on how many rows run beside it:
+    12 rows (16-row weight tiles in every linear) against the same rows four at a
+    time (8-row tiles).  Each is within 1e-2 of the exact logits."""
+    W = lib.s2pfa_weights_of(decoder[0] if isinstance(decoder, tuple) else decoder)
+    big = ctypes.c_void_p()
+    s2pamd.check(lib.s2pfa_create(ctypes.byref(big), W, 12, S()), "fastar create")
+    try:
+        r = np.random.default_rng(12)
+        hid = to_dev(bf16_bits(r.standard_normal((12, DIM)).astype(np.float32)))
+        sem = to_dev(r.integers(0, CB, 12).astype(np.int32))
+        stage = ctypes.c_void_p()
+
+        def frame(h, s, n):
+            lg = empty((9, n, CB))
+            s2pamd.check(lib.s2pfa_decode_frame_logits_dev(big, P(h), P(s), n, ctypes.byref(stage),
+                                                           P(lg), S()), "frame")
+            return bf16_vals(to_host(lg, np.uint16))[0].astype(np.float64)
+
+        whole = frame(hid, sem, 12)
+        for i in range(0, 12, 4):
+            part = frame(hid[i:i + 4].contiguous(), sem[i:i + 4].contiguous(), 4)
+            d = np.linalg.norm(whole[i:i + 4] - part, axis=1) / np.linalg.norm(part, axis=1)
+            assert (d <= 2e-2).all(), (i, d)
+    finally:
+        sync()
+        lib.s2pfa_free(big)

@@ -102,6 +102,50 @@ def test_int4p_gemm_six_tiles_repeat(lib, M, N, K):
             assert bad.size == 0, f"call {i}: {len(bad)} outputs differ, first at {bad[:4].tolist()}"
 
 
+# M <= 16: both tile widths (8 and 16 rows) at their edges, rows and tiles that
+# do not divide, the streamed and the resident K classes, K with idle waves
+@pytest.mark.parametrize("fmt", ["int4", "int8", "bf16"])
+@pytest.mark.parametrize("N,K", [(5, 2560), (4097, 2560), (19461, 2560), (2567, 4096),
+                                 (2560, 9728), (4103, 9728), (33, 512), (9, 1024)])
+def test_gemv_small_m(lib, fmt, N, K):
+    r = np.random.default_rng(N + K)
+    if fmt == "int4":
+        w, s = rand_int4(r, N, K)
+        s[0, K // 64] = 0x7C00  # an infinite group scale stays in its own row
+        b = w.astype(np.int8)
+        q = np.stack([(b << 4).astype(np.int8) >> 4, b >> 4], -1).reshape(N, K // 32, 32)
+        sf = s.view(np.float16).astype(np.float64)
+        sf[0] = 0.0
+        wf = (q * sf[:, :, None]).reshape(N, K)
+    elif fmt == "int8":
+        w = r.integers(-128, 128, (N, K)).astype(np.int8)
+        s = (np.abs(r.standard_normal(N)) * 0.01).astype(np.float32)
+        wf = w.astype(np.float64) * s[:, None].astype(np.float64)
+    else:
+        w, s = bf16_bits(r.standard_normal((N, K)).astype(np.float32) / np.sqrt(K)), None
+        wf = bf16_vals(w).astype(np.float64)
+    xh = bf16_bits(r.standard_normal((16, K)).astype(np.float32))
+    wd, sd, xd = to_dev(w), None if s is None else to_dev(s), to_dev(xh)
+    exact = bf16_vals(xh).astype(np.float64) @ wf.T
+    for M in (1, 4, 8, 9, 16):
+        y = empty((M, N))
+        if fmt == "int4":
+            rc = lib.s2p_int4p_gemv(P(y), P(xd), P(wd), P(sd), M, N, K, 32, S())
+        elif fmt == "int8":
+            rc = lib.s2p_int8_gemv(P(y), P(xd), P(wd), P(sd), M, N, K, S())
+        else:
+            rc = lib.s2p_gemm_bf16(P(xd), P(wd), P(y), M, N, K, S())
+        s2pamd.check(rc, fmt)
+        got = bf16_vals(to_host(y, np.uint16)).astype(np.float64)
+        if fmt == "int4":
+            assert not np.isfinite(got[:, 0]).any()
+            got[:, 0] = 0.0
+        # one bf16 rounding (2^-9) of an f32 sum whose terms round at 2^-24 of
+        # the row's magnitude
+        bound = 2.0 ** -8 * np.abs(exact[:M]) + 1e-4 * np.abs(exact[:M]).max(1, keepdims=True)
+        assert (np.abs(got - exact[:M]) <= bound).all(), (fmt, M, N, K)
+
+
 def test_int4p_gemv_closed_forms(lib, engine):
     """All weights -8, unit scales: y = -8 * sum(x); single nonzero weight."""
     M, N, K = 4, 64, 2560
