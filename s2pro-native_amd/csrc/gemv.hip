@@ -54,9 +54,9 @@
 #include "gemv_dev.h"
 #include "s2pro/gemm.h"
 
-/* whole-K workgroups of up to 16 waves (MT = 1) or 8 waves */
-template <int WFMT, int MT, bool NOTR = false>
-__global__ __launch_bounds__(MT == 1 ? 1024 : 512) void k_gemv3(GemvArgs a) {
+/* whole-K workgroups of up to 16 waves, one column tile (M <= 16) */
+template <int WFMT>
+__global__ __launch_bounds__(1024) void k_gemv3(GemvArgs a) {
     extern __shared__ __align__(16) unsigned char smem3[];
     /* every argument in one round of scalar loads: left to itself the
      * compiler issues them next to their first uses, three dependent
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void k_gemv3(GemvArgs a) {
                  "s"(a.K), "s"(a.gps), "s"(a.ks), "s"(a.rt), "s"(a.xmode), "s"(a.epi),
                  "s"(a.ssq_in_blocks), "s"(a.norm_eps), "s"(gridDim.x));
     GvBuf b0, b1;
-    gv3_block<WFMT, MT, false, false, false, NOTR>(a, blockIdx.x, gridDim.x,
+    gv3_block<WFMT, 1, false, false, false, false>(a, blockIdx.x, gridDim.x,
                                                   (LDS(unsigned char)*)smem3, a.y, b0, b1);
 }
 
@@ -241,11 +241,11 @@ extern "C" hipError_t s2p_gemv_plan(GemvArgs* ap, int slots, dim3* grid_out, siz
  * hipErrorNotSupported when the activations do not fit in LDS (the split-K
  * engine runs instead). */
 extern "C" hipError_t s2p_gemv3_plan(GemvArgs* a, dim3* grid, dim3* block, size_t* lds_out) {
+    if (a->M > 16) return hipErrorNotSupported;
     const int G = a->K >> 5;
-    const int mt = (a->M + 15) / 16;
     const bool swiglu = a->epi == GEMV_EPI_SWIGLU;
     const int tiles = swiglu ? (a->N >> 1) / 16 : (a->N + 15) / 16;
-    const int nwmax = mt == 1 ? 16 : 8;
+    const int nwmax = 16;
     const int chg = gv_chg(a->wfmt);
     const int cus = s2p_cu_count();
     const int kmax = swiglu ? nwmax / 2 : nwmax;
@@ -268,7 +268,7 @@ extern "C" hipError_t s2p_gemv3_plan(GemvArgs* a, dim3* grid, dim3* block, size_
         const int rt = per * units, nw = rt * ks;
         const int ngroups = (tiles + units - 1) / units;
         /* resident workgroups per CU: LDS, and waves at this kernel's
-         * register budget (16 waves per CU at MT = 1, else 8) */
+         * register budget (16 waves per CU) */
         const size_t lds1 = gv3_lds_bytes(a->M, gps, a->wfmt, ks, nw, 1);
         int per_cu = (int)(GV3_LDS_MAX / lds1);
         const int wcap = nwmax / nw;
@@ -292,37 +292,16 @@ extern "C" hipError_t s2p_gemv3_plan(GemvArgs* a, dim3* grid, dim3* block, size_
     }
 }
 
-template <int WFMT, int MT, bool NOTR>
-static hipError_t gv3_launch_k(const GemvArgs& a, dim3 grid, dim3 block, size_t lds,
-                               hipStream_t st) {
-    /* once per instantiation (thread-safe static initialisation) */
-    static const hipError_t attr = hipFuncSetAttribute((const void*)k_gemv3<WFMT, MT, NOTR>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       GV3_LDS_MAX);
-    (void)attr;
-    hipLaunchKernelGGL((k_gemv3<WFMT, MT, NOTR>), grid, block, lds, st, a);
-    return hipGetLastError();
-}
-
-template <int WFMT, int MT>
-static hipError_t gv3_launch_mt(const GemvArgs& a, dim3 grid, dim3 block, size_t lds,
-                                hipStream_t st) {
-    return gv3_launch_k<WFMT, MT, false>(a, grid, block, lds, st);
-}
-
 template <int WFMT>
 static hipError_t gv3_launch(const GemvArgs& a, dim3 grid, dim3 block, size_t lds,
                              hipStream_t st) {
-    switch ((a.M + 15) / 16) {
-        case 1: return gv3_launch_mt<WFMT, 1>(a, grid, block, lds, st);
-        case 2: return gv3_launch_mt<WFMT, 2>(a, grid, block, lds, st);
-        case 3: return gv3_launch_mt<WFMT, 3>(a, grid, block, lds, st);
-        case 4: return gv3_launch_mt<WFMT, 4>(a, grid, block, lds, st);
-        case 5: return gv3_launch_mt<WFMT, 5>(a, grid, block, lds, st);
-        case 6: return gv3_launch_mt<WFMT, 6>(a, grid, block, lds, st);
-        case 7: return gv3_launch_mt<WFMT, 7>(a, grid, block, lds, st);
-        default: return gv3_launch_mt<WFMT, 8>(a, grid, block, lds, st);
-    }
+    /* once per instantiation (thread-safe static initialisation) */
+    static const hipError_t attr = hipFuncSetAttribute((const void*)k_gemv3<WFMT>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       GV3_LDS_MAX);
+    (void)attr;
+    hipLaunchKernelGGL((k_gemv3<WFMT>), grid, block, lds, st, a);
+    return hipGetLastError();
 }
 
 static hipError_t gemv_engines(const GemvArgs* ap, hipStream_t st) {
@@ -334,7 +313,7 @@ static hipError_t gemv_engines(const GemvArgs* ap, hipStream_t st) {
         dim3 block;
         const hipError_t e3 = s2p_gemv_plan_check(&a3);
         if (e3 != hipSuccess) return e3;
-        if (a.M <= 16) { /* loads in the operand layout, every load in flight (gemvr.hip) */
+        if (a.M <= 16 && a.engine == GEMV_ENGINE_AUTO) { /* loads in the operand layout, every load in flight (gemvr.hip) */
             const hipError_t er = s2p_gvr_launch(&a, st);
             if (er != hipErrorNotSupported) return er;
         }
@@ -377,13 +356,20 @@ static hipError_t gemv_engines(const GemvArgs* ap, hipStream_t st) {
 
 extern "C" hipError_t s2p_gemv_launch(const GemvArgs* ap, hipStream_t st) {
     if (ap->deferred) *ap->deferred = 0; /* merged, unless k_gemm4 defers below */
-    /* INT4 at 16 < M <= 96: the row-split GEMM with streamed activation
-     * windows (gemm4.hip), which writes inv_out itself */
-    if (ap->engine == GEMV_ENGINE_AUTO && ap->gps == 0 && ap->wfmt == GEMV_W_INT4 && ap->M > 16) {
-        const hipError_t e4 = s2p_gemm4_launch(ap, st);
-        if (e4 != hipErrorNotSupported) return e4;
+    hipError_t e = hipErrorNotSupported;
+    if (ap->engine != GEMV_ENGINE_SPLITK && ap->gps == 0 && ap->M > 16) {
+        e = s2p_gemv_plan_check(ap);
+        if (e != hipSuccess) return e;
+        /* packed activations, register operands (gemmx.hip) */
+        e = ap->engine == GEMV_ENGINE_AUTO ? s2p_gmx_launch(ap, st) : hipErrorNotSupported;
+        if (e == hipErrorNotSupported && ap->wfmt == GEMV_W_INT4) {
+            /* the row-split GEMM with streamed activation windows (gemm4.hip),
+             * which writes inv_out itself */
+            const hipError_t e4 = s2p_gemm4_launch(ap, st);
+            if (e4 != hipErrorNotSupported) return e4;
+        }
     }
-    const hipError_t e = gemv_engines(ap, st);
+    if (e == hipErrorNotSupported) e = gemv_engines(ap, st);
     /* the inverse RMS is read by k_gemm4 only, whose rows are the same M */
     if (e != hipSuccess || ap->M <= 16 || !ap->inv_out || ap->epi != GEMV_EPI_RESID || !ap->ssq_out)
         return e;

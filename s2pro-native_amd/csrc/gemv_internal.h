@@ -19,7 +19,7 @@ enum { GEMV_X_PLAIN = 0, GEMV_X_NORM = 1 };            /* activation staging */
  * sums of squares; SWIGLU: W = [gate; up] (2F rows), y[m][F] =
  * silu(bf16(gate)) * bf16(up) with the rule's roundings. */
 enum { GEMV_EPI_STORE = 0, GEMV_EPI_RESID = 1, GEMV_EPI_SWIGLU = 2 };
-enum { GEMV_ENGINE_AUTO = 0, GEMV_ENGINE_SPLITK = 2 };
+enum { GEMV_ENGINE_AUTO = 0, GEMV_ENGINE_STAGED = 1, GEMV_ENGINE_SPLITK = 2 };
 
 typedef struct {
     const uint8_t*  w;       /* INT4: packed [N][K/2]; INT8: [N][K]; BF16: bf16 [N][K] */
@@ -46,7 +46,9 @@ typedef struct {
     float*          part;    /* [splits][M][nrb][64] fp32 */
     int64_t         part_cap;/* floats available at part */
     unsigned*       counters;/* [ceil(N/64)], zero between calls */
-    int             engine;  /* GEMV_ENGINE_AUTO, or GEMV_ENGINE_SPLITK: the split-K engine only */
+    int             engine;  /* GEMV_ENGINE_AUTO; GEMV_ENGINE_STAGED: the engines that stage their
+                              * activations in LDS (k_gemv3, k_gemm4) where they take the shape;
+                              * GEMV_ENGINE_SPLITK: the split-K engine only */
     const float*    inv_in;  /* NORM (k_gemm4): the rows' inverse RMS, [M], when the producer
                               * wrote it (NULL: computed here) */
     float*          inv_out; /* RESID: also write the output rows' inverse RMS, [M] (NULL: no) */
@@ -61,6 +63,8 @@ typedef struct {
 } GemvArgs;
 
 hipError_t s2p_gemv_launch(const GemvArgs* a, hipStream_t st);
+/* 16 < M <= 128 (gemmx.hip); hipErrorNotSupported outside its shapes */
+hipError_t s2p_gmx_launch(const GemvArgs* a, hipStream_t st);
 /* INT4, 16 < M <= 96 (gemm4.hip); hipErrorNotSupported outside that range */
 hipError_t s2p_gemm4_launch(const GemvArgs* a, hipStream_t st);
 /* M <= 16 (gemvr.hip); hipErrorNotSupported outside its shapes */

@@ -653,7 +653,7 @@ static hipError_t gr_nt(const GvrArgs& a, int nt, int grid, hipStream_t st) {
 
 /* resident classes, the model's widths (every wave the same number U of whole
  * units, no checks between the tiles' multiplies): 1: K = 2560 on 10 waves;
- * 2: K = 4096 on 8.  Any other K streams.  NT / NTW / NTN: most tiles a round that
+ * 2: K = 4096 on 8.  A longer K streams.  NT / NTW / NTN: most tiles a round that
  * the registers hold, narrow / WIDE / WIDE with a norm.  U3: units a wave of
  * 16 waves that hold a longer K (w2's 9728) whole, two tiles, one round */
 template <int WFMT>
@@ -677,7 +677,9 @@ static hipError_t gr_launch(GvrArgs& a, bool norm, hipStream_t st) {
     const int units = a.K / gr_uk(WFMT), cus = s2p_cu_count();
     const bool swiglu = a.epi == GEMV_EPI_SWIGLU;
     const int cls = units == 10 * Cl::U1 ? 1 : units == 8 * Cl::U2 ? 2 : 0;
-    if ((norm && cls != 1) || (swiglu && cls == 0)) return hipErrorNotSupported;
+    /* only a long K streams: at K = 1024 its rounds of 16 rows took 18 us where
+     * the staged engine takes 8 (INT4, 18742 rows, M = 2) */
+    if ((norm && cls != 1) || (cls == 0 && (swiglu || a.K <= 4096))) return hipErrorNotSupported;
     const int per = swiglu ? 2 : 1; /* weight tiles per output tile */
     const int rows = swiglu ? a.N >> 1 : a.N, trows = gr_rows(WIDE);
     int most = (cls == 1   ? (!WIDE ? Cl::NT1 : norm ? Cl::NTN1 : Cl::NTW1)

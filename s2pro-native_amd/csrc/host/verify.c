@@ -507,12 +507,17 @@ static void gemv_args(GemvArgs* ap, const s2p_linear* lin, int M, const void* x,
 /* inv_out / inv_in: the output rows' inverse RMS written by a residual GEMV
  * for the normed GEMV that reads them next (the row-split INT4 GEMM at
  * 16 < M <= 96 only: elsewhere the consumer computes its own) */
-static s2p_status gemv_ex(const s2p_linear* lin, int M, const void* x, int ldx, void* y,
+static s2p_status gemv_ex(const s2p_backbone* b, const s2p_linear* lin, int M, const void* x, int ldx, void* y,
                           int ldy, int xmode, const void* norm_w, const float* ssq_in, int epi,
                           float* ssq_out, const float* inv_in, float* inv_out,
                           S2pQkvParts* parts, hipStream_t st) {
     GemvArgs a;
     gemv_args(&a, lin, M, x, ldx, y, ldy, xmode, norm_w, ssq_in, epi, ssq_out);
+    /* An appended INT8 / INT4 code is a rounded sum: another summation order
+     * moves about 5% of the codes from the second layer on (measured, 16
+     * rows, two layers).  Plans over quantised caches keep the engines, and
+     * the order, that the codes already in such caches were written with */
+    if (b->kvb != 16 && lin->q_packed) a.engine = GEMV_ENGINE_STAGED;
     int deferred = 0;
     if (M > 16 && M <= 96) {
         a.inv_in = inv_in;
@@ -530,10 +535,10 @@ static s2p_status gemv_ex(const s2p_linear* lin, int M, const void* x, int ldx, 
     return S2P_OK;
 }
 
-static s2p_status gemv(const s2p_linear* lin, int M, const void* x, int ldx, void* y, int ldy,
+static s2p_status gemv(const s2p_backbone* b, const s2p_linear* lin, int M, const void* x, int ldx, void* y, int ldy,
                        int xmode, const void* norm_w, const float* ssq_in, int epi, float* ssq_out,
                        const float* inv_in, float* inv_out, hipStream_t st) {
-    return gemv_ex(lin, M, x, ldx, y, ldy, xmode, norm_w, ssq_in, epi, ssq_out, inv_in, inv_out,
+    return gemv_ex(b, lin, M, x, ldx, y, ldy, xmode, norm_w, ssq_in, epi, ssq_out, inv_in, inv_out,
                    NULL, st);
 }
 
@@ -651,6 +656,9 @@ s2p_status s2p_verify_forward(s2p_backbone* b, const void* x_in, void* logits, h
     float* ssq_b = b->ssq + (S2P_DIM / GEMV_SSQ_COLS) * GEMV_MAX_M;
     float* inv_a = b->ssq + 2 * (S2P_DIM / GEMV_SSQ_COLS) * GEMV_MAX_M;
     float* inv_b = inv_a + GEMV_MAX_M;
+    /* the inverse RMS goes from a residual GEMM to the next norm where both run
+     * on k_gemm4; the other engines take it from the rows themselves */
+    if (b->o.quant != S2P_WQ_INT4_G32 || M <= 16 || M > 96) inv_a = inv_b = NULL;
     S2P_TRY(hip_ok(s2p_resid_init_launch(x_in, b->x, ssq_a, M, S2P_DIM, st), "resid init"));
     for (int l = 0; l < b->o.n_layers; l++) {
         const s2p_slow_layer* L = &b->layers[l];
@@ -659,7 +667,7 @@ s2p_status s2p_verify_forward(s2p_backbone* b, const void* x_in, void* logits, h
          * attention prologue of the other plans measured slower reading them:
          * every split's blocks reread the partials) */
         S2pQkvParts qp = {NULL, 0, 0, 0};
-        S2P_TRY(gemv_ex(&L->wqkv, M, b->x, S2P_DIM, b->qkv, S2P_QKV_WIDTH, GEMV_X_NORM,
+        S2P_TRY(gemv_ex(b, &L->wqkv, M, b->x, S2P_DIM, b->qkv, S2P_QKV_WIDTH, GEMV_X_NORM,
                         L->attn_norm.data, ssq_a, GEMV_EPI_STORE, NULL, l > 0 ? inv_a : NULL,
                         NULL, b->kvb == 16 && b->tree ? &qp : NULL, st));
         if (b->kvb != 16) {
@@ -688,14 +696,14 @@ s2p_status s2p_verify_forward(s2p_backbone* b, const void* x_in, void* logits, h
                                                   L->q_norm.data, L->k_norm.data, b->d_rope,
                                                   NORM_EPS, NULL, st),
                        "attention"));
-        S2P_TRY(gemv(&L->wo, M, b->attn, S2P_Q_HEADS * S2P_HEAD_DIM, b->x, S2P_DIM, GEMV_X_PLAIN,
+        S2P_TRY(gemv(b, &L->wo, M, b->attn, S2P_Q_HEADS * S2P_HEAD_DIM, b->x, S2P_DIM, GEMV_X_PLAIN,
                      NULL, NULL, GEMV_EPI_RESID, ssq_b, NULL, inv_b, st));
-        S2P_TRY(gemv(&L->gate_up, M, b->x, S2P_DIM, b->gu, S2P_FFN_DIM, GEMV_X_NORM,
+        S2P_TRY(gemv(b, &L->gate_up, M, b->x, S2P_DIM, b->gu, S2P_FFN_DIM, GEMV_X_NORM,
                      L->ffn_norm.data, ssq_b, GEMV_EPI_SWIGLU, NULL, inv_b, NULL, st));
-        S2P_TRY(gemv(&L->w2, M, b->gu, S2P_FFN_DIM, b->x, S2P_DIM, GEMV_X_PLAIN, NULL, NULL,
+        S2P_TRY(gemv(b, &L->w2, M, b->gu, S2P_FFN_DIM, b->x, S2P_DIM, GEMV_X_PLAIN, NULL, NULL,
                      GEMV_EPI_RESID, ssq_a, NULL, inv_a, st));
     }
-    return gemv(&b->head, M, b->x, S2P_DIM, logits, b->head.out_features, GEMV_X_NORM,
+    return gemv(b, &b->head, M, b->x, S2P_DIM, logits, b->head.out_features, GEMV_X_NORM,
                 b->final_norm.data, ssq_a, GEMV_EPI_STORE, NULL, b->o.n_layers > 0 ? inv_a : NULL,
                 NULL, st);
 }

@@ -146,6 +146,48 @@ def test_gemv_small_m(lib, fmt, N, K):
         assert (np.abs(got - exact[:M]) <= bound).all(), (fmt, M, N, K)
 
 
+# 16 < M <= 128 through s2p_linear_forward: edges of the activation tiles (wave
+# groups of one, two and four), rows that do not divide, K splits and none
+@pytest.mark.parametrize("fmt", ["int4", "int8", "bf16"])
+@pytest.mark.parametrize("N,K", [(12289, 512), (4097, 2560), (70, 1152), (2567, 9728), (5, 128),
+                                 (40003, 256)])
+def test_linear_large_m(lib, fmt, N, K):
+    r = np.random.default_rng(N * 3 + K)
+    lin = s2pamd.Linear()
+    lin.in_features, lin.out_features = K, N
+    if fmt == "int4":
+        w, s = rand_int4(r, N, K)
+        b = w.astype(np.int8)
+        q = np.stack([(b << 4).astype(np.int8) >> 4, b >> 4], -1).reshape(N, K // 32, 32)
+        wf = (q * s.view(np.float16).astype(np.float64)[:, :, None]).reshape(N, K)
+        wd, sd = to_dev(w), to_dev(s)
+        lin.w_pack.data, lin.q_packed, lin.q_group = wd.data_ptr(), 1, 32
+    elif fmt == "int8":
+        w = r.integers(-128, 128, (N, K)).astype(np.int8)
+        s = (np.abs(r.standard_normal(N)) * 0.01).astype(np.float32)
+        wf = w * s[:, None].astype(np.float64)
+        wd, sd = to_dev(w), to_dev(s)
+        lin.w_int8.data = wd.data_ptr()
+    else:
+        w = bf16_bits(r.standard_normal((N, K)).astype(np.float32) / np.sqrt(K))
+        wf, wd, sd = bf16_vals(w).astype(np.float64), to_dev(w), None
+        lin.w_bf16.data = wd.data_ptr()
+    if sd is not None:
+        lin.w_iscale.data, lin.int8_ready = sd.data_ptr(), 1
+    xh = bf16_bits(r.standard_normal((128, K)).astype(np.float32))
+    xd = to_dev(xh)
+    exact = bf16_vals(xh).astype(np.float64) @ wf.T
+    for M in (17, 48, 49, 65, 96, 97, 113, 128):
+        y = empty((M, N))
+        s2pamd.check(lib.s2p_linear_forward(ctypes.byref(lin), P(xd), P(y), M,
+                                            0 if fmt == "bf16" else 2, S()), fmt)
+        got = bf16_vals(to_host(y, np.uint16)).astype(np.float64)
+        # one bf16 rounding (2^-9) of an f32 sum whose terms round at 2^-24 of
+        # the row's magnitude
+        bound = 2.0 ** -8 * np.abs(exact[:M]) + 1e-4 * np.abs(exact[:M]).max(1, keepdims=True)
+        assert (np.abs(got - exact[:M]) <= bound).all(), (fmt, M, N, K)
+
+
 def test_int4p_gemv_closed_forms(lib, engine):
     """All weights -8, unit scales: y = -8 * sum(x); single nonzero weight."""
     M, N, K = 4, 64, 2560

@@ -439,3 +439,30 @@ def test_verify_plan_device_tree(lib):
         assert np.array_equal(got_a, got_b)
     finally:
         lib.s2p_backbone_free(bb)
+
+
+def test_int8_layers_int4_head_batch(lib):
+    """INT8 layers under an INT4 head at 20 rows (two GEMM engines in one
+    forward, the head's norm on the layers' sums of squares) give every session
+    the logits it gets alone at 5 rows; each is within 1e-2 of the exact ones."""
+    n, R, L, ctx = 4, 5, 70, 128
+    o = s2pamd.BackboneOpts(1, s2pamd.WQ_INT8, s2pamd.WQ_INT4, s2pamd.S2P_HEAD_SLICE, n * R, n, ctx, 0)
+    bb = ctypes.c_void_p()
+    s2pamd.check(lib.s2p_backbone_create_random(ctypes.byref(o), 31, S(), ctypes.byref(bb)))
+    try:
+        parent = [-1, 0, 1, 2, 3]
+        kvs = [new_kv(lib, bb, 50 + i) for i in range(n)]
+        x = to_dev(bf16_bits(np.random.default_rng(8).standard_normal((n * R, 2560)).astype(np.float32)))
+
+        def run(xs, sel):
+            plan(lib, bb, parent, [kvs[i] for i in sel], [L - i for i in sel])
+            lg = empty((len(sel) * R, s2pamd.S2P_HEAD_SLICE))
+            s2pamd.check(lib.s2p_verify_forward(bb, P(xs), P(lg), S()))
+            return bf16_vals(to_host(lg, np.uint16)).astype(np.float64)
+
+        whole = run(x, list(range(n)))
+        for i in range(n):
+            part = run(x[i * R:(i + 1) * R].contiguous(), [i])
+            assert_close_norm(whole[i * R:(i + 1) * R], part, rel=2e-2, what=f"session {i}")
+    finally:
+        lib.s2p_backbone_free(bb)
