@@ -4,7 +4,8 @@
  * and split-K flash-decode (kernels.cu:341-508), and adds the tree mask the
  * verify pass needs.  One kernel serves three callers:
  *   CONTIG  s2pk_attention: one contiguous cache, rows at positions pos..;
- *   PTRS    s2pk_attention_ptrs / _decode: per-row caches and positions;
+ *   PTRS    s2pk_attention_ptrs: per-row caches and positions (decode with the
+ *           longest session known to the host is attn_decode.hip);
  *   PLAN    the verify forward: sessions x rows with per-row visibility
  *           masks (causal chain or draft tree) relative to the prefix L.
  *
@@ -412,6 +413,13 @@ extern "C" hipError_t s2pk_attention_ptrs(const s2p_bf16* q, const s2p_bf16* con
     return attn_run(a, rows, 1, max_seq, 0, st);
 }
 
+/* attn_decode.hip */
+extern "C" hipError_t s2p_attn_dec_launch(const uint16_t* q, const void* const* kcs,
+                                          const void* const* vcs, const uint16_t* const* kss,
+                                          const uint16_t* const* vss, uint16_t* out, int rows,
+                                          int kv_heads, const int32_t* pos, int max_seq,
+                                          int max_len, float* part, int bw, hipStream_t st);
+
 extern "C" int64_t s2pk_attention_part_floats(int rows, int q_heads, int max_len) {
     const int nsplit = (max_len + AT_TILE * AT_WAVES - 1) / (AT_TILE * AT_WAVES);
     return part_floats(rows, q_heads, nsplit < 1 ? 1 : nsplit);
@@ -425,19 +433,9 @@ extern "C" hipError_t s2pk_attention_decode(const s2p_bf16* q, const s2p_bf16* c
     if (rows <= 0) return hipSuccess;
     if (head_dim != AT_HD || q_heads != 4 * kv_heads || !part || max_len <= 0)
         return hipErrorInvalidValue;
-    AttnArgs a = {};
-    a.mode = AM_PTRS;
-    a.q = (const uint16_t*)q;
-    a.out = (uint16_t*)out;
-    a.rows = rows;
-    a.qh = q_heads;
-    a.kvh_n = kv_heads;
-    a.kcs = (const uint16_t* const*)k_caches;
-    a.vcs = (const uint16_t* const*)v_caches;
-    a.pos = pos;
-    a.max_seq = max_seq;
-    a.part = part;
-    return attn_run(a, rows, 1, max_len, s2pk_attention_part_floats(rows, q_heads, max_len), st);
+    return s2p_attn_dec_launch((const uint16_t*)q, (const void* const*)k_caches,
+                               (const void* const*)v_caches, nullptr, nullptr, (uint16_t*)out,
+                               rows, kv_heads, pos, max_seq, max_len, part, 16, st);
 }
 
 extern "C" int64_t s2p_attn_plan_part_floats(int rows, int max_span) {

@@ -219,6 +219,12 @@ __global__ __launch_bounds__(KV8_TILE) void k_attention8_split(
 extern "C" hipError_t s2p_attn_combine_launch(const float* part, uint16_t* out, int rows, int qh,
                                               int nsplit, hipStream_t st);
 
+extern "C" hipError_t s2p_attn_dec_launch(const uint16_t* q, const void* const* kcs,
+                                          const void* const* vcs, const uint16_t* const* kss,
+                                          const uint16_t* const* vss, uint16_t* out, int rows,
+                                          int kv_heads, const int32_t* pos, int max_seq,
+                                          int max_len, float* part, int bw, hipStream_t st);
+
 extern "C" hipError_t s2pk_kv_append8(const s2p_bf16* k, const s2p_bf16* v, int8_t* k_cache,
                                       int8_t* v_cache, void* k_scale, void* v_scale, int rows,
                                       int kv_heads, int head_dim, int pos, int max_seq, int bw,
@@ -293,6 +299,11 @@ extern "C" hipError_t s2pk_attention8_decode(const s2p_bf16* q, const int8_t* co
     if (head_dim != KV8_HD || (bw != 8 && bw != 4) || kv_heads <= 0 || q_heads % kv_heads ||
         !part || max_len <= 0 || !pos)
         return hipErrorInvalidValue;
+    if (q_heads == 4 * kv_heads) /* the model's grouping (attn_decode.hip) */
+        return s2p_attn_dec_launch((const uint16_t*)q, (const void* const*)k_caches,
+                                   (const void* const*)v_caches, (const uint16_t* const*)k_scales,
+                                   (const uint16_t* const*)v_scales, (uint16_t*)out, rows, kv_heads,
+                                   pos, max_seq, max_len, part, bw, st);
     const int nsplit = (max_len + KV8_TILE - 1) / KV8_TILE;
     const dim3 grid((unsigned)rows, (unsigned)q_heads, (unsigned)nsplit);
     if (bw == 8)

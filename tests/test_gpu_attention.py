@@ -3,6 +3,7 @@ GPU kernel uses MFMA with bf16 probabilities; the oracle restates the
 reference's fp32 order, or_attention / or_attention_split)."""
 import numpy as np
 import pytest
+import torch
 
 import pyoracle as po
 import s2pamd
@@ -183,3 +184,63 @@ def test_attention_tree_kernel(lib, R, Ls, max_seq):
         err = np.abs(got[s * R:(s + 1) * R] - exact)
         assert err.max() < 2e-2, (f"session {s}: max err {err.max():.4g} at "
                                   f"{np.unravel_index(err.argmax(), err.shape)}")
+
+
+# tile (32 slots), wave round (128) and split edges, one split and many; a row
+# outside its cache sees nothing and leaves the others alone; scores of -inf
+# weigh nothing; payloads and scales at odd addresses
+@pytest.mark.parametrize("bw", [16, 8, 4])
+@pytest.mark.parametrize("lens", [[1], [1, 31, 33, 127, 128], [129, 32, 515, 1, 260, 384, 97],
+                                  [2049, 64]])
+def test_attention_decode_edges(lib, bw, lens):
+    r = np.random.default_rng(len(lens) * 100 + bw)
+    n, cap, mx = len(lens), max(lens) + 3, max(lens)
+    q = r.standard_normal((n + 1, 32, 128)).astype(np.float32)
+    q[:, :4, 0] = 1.0
+    qd = to_dev(bf16_bits(q))
+
+    def off_by(a, by):  # a's bytes on the device, `by` past an aligned address
+        return to_dev(np.concatenate([np.zeros(by, np.uint8), a.view(np.uint8).ravel()]))[by:]
+
+    ks, vs, kd, vd, ksd, vsd = [], [], [], [], [], []
+    for i in range(n + 1):
+        vals = []
+        for dst, sdst in ((kd, ksd), (vd, vsd)):
+            if bw == 16:
+                x = r.standard_normal((8, cap, 128)).astype(np.float32)
+                if dst is kd and i < n and lens[i] > 32:
+                    x[0, :32, 0] = -np.inf  # a whole tile of kv head 0
+                x = bf16_bits(x)
+                dst.append(to_dev(x))
+                vals.append(bf16_vals(x).astype(np.float64))
+                continue
+            lim = 127 if bw == 8 else 7
+            c = r.integers(-lim, lim + 1, (8, cap, 128)).astype(np.int8)
+            s = (np.abs(r.standard_normal((8, cap, 4))) * (1.5 / lim)).astype(np.float16)
+            packed = c if bw == 8 else (c[..., 0::2] & 15) | ((c[..., 1::2] & 15) << 4)
+            dst.append(off_by(np.ascontiguousarray(packed.astype(np.int8)), 1))
+            sdst.append(off_by(s, 2))
+            vals.append(c.astype(np.float64) * np.repeat(s.astype(np.float64), 32, axis=2))
+        ks.append(vals[0])
+        vs.append(vals[1])
+    ptr = lambda ts: to_dev(np.array([t.data_ptr() for t in ts], np.int64))
+    pos = to_dev(np.array([v - 1 for v in lens] + [cap], np.int32))  # the last row: outside
+    part = empty((lib.s2pk_attention_part_floats(n + 1, 32, mx),), torch.float32)
+    out = empty((n + 1, 32 * 128))
+    if bw == 16:
+        rc = lib.s2pk_attention_decode(P(qd), P(ptr(kd)), P(ptr(vd)), P(out), n + 1, 32, 8, 128,
+                                       P(pos), cap, mx, P(part), S())
+    else:
+        rc = lib.s2pk_attention8_decode(P(qd), P(ptr(kd)), P(ptr(vd)), P(ptr(ksd)), P(ptr(vsd)),
+                                        P(out), n + 1, 32, 8, 128, P(pos), cap, mx, P(part), bw, S())
+    s2pamd.hip_check(rc, "decode")
+    got = bf16_vals(to_host(out, np.uint16)).reshape(n + 1, 32, 128).astype(np.float64)
+    for i, L in enumerate(lens):
+        qi = bf16_vals(bf16_bits(q[i])).astype(np.float64)
+        for h in range(32):
+            sc = ks[i][h // 4, :L] @ qi[h] / np.sqrt(128.0)
+            p = np.exp(sc - sc.max())
+            want = (p / p.sum()) @ vs[i][h // 4, :L]
+            # one bf16 rounding (2^-9) of an f32 sum, f32 exponentials
+            bound = 2.0 ** -8 * np.abs(want) + 2e-4 * np.abs(vs[i][h // 4, :L]).max()
+            assert (np.abs(got[i, h] - want) <= bound).all(), (bw, L, h)
