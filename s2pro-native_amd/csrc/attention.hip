@@ -3,7 +3,8 @@
  * Replaces the reference's causal single-pass attention (kernels.cu:234-339)
  * and split-K flash-decode (kernels.cu:341-508), and adds the tree mask the
  * verify pass needs.  One kernel serves three callers:
- *   CONTIG  s2pk_attention: one contiguous cache, rows at positions pos..;
+ *   CONTIG  s2pk_attention: one contiguous cache, rows at positions pos..
+ *           (8 waves a block, no scratch and so no position splits);
  *   PTRS    s2pk_attention_ptrs: per-row caches and positions (decode with the
  *           longest session known to the host is attn_decode.hip);
  *   PLAN    the verify forward: sessions x rows with per-row visibility
@@ -30,17 +31,22 @@
 #include <stdint.h>
 
 #include "attn_dev.h"
+#include "gemv_internal.h"
 #include "s2pro/kernels.h"
 #include "s2pro/slowar_kernels.h"
 
 /* Position splits are sized so that the grid stays within AT_MAX_BLOCKS
  * blocks (two per CU): a block's fixed costs (q load or the fused prologue,
- * the wave merge, the partial store) are paid once per block, so at configs
- * 4 / 5 (8 x 4096 / 4 x 8192 positions) 512 blocks ran the layer's
+ * the wave merge, the partial store) are paid once per block, so at 8 x 4096
+ * and 4 x 8192 positions 512 blocks ran the layer's
  * attention in 34 / 85 us against 54 / 112 us with 4096. */
 #ifndef AT_MAX_BLOCKS
 #define AT_MAX_BLOCKS 512
 #endif
+/* segments up to which the splits are balanced: beyond half the 64 blocks of
+ * a kv head there is little left to divide */
+#define AT_BAL_SEGS 32
+#define AT_ROUND (AT_TILE * AT_WAVES) /* positions a block of AT_WAVES waves takes at a time */
 
 /* Blocks are numbered (segment fastest, then kv head, then split) and the
  * numbering is laid over the 8 XCDs in contiguous chunks: workgroup i runs
@@ -57,21 +63,71 @@ extern "C" hipError_t s2p_at_probe_get(uint64_t* host, int n) {
 }
 #endif
 
+/* The balanced splits of a plan's segments (one segment a lane, n_seg <= 64):
+ * every segment is cut into splits of u rounds (a round is 128 positions, a
+ * tile a wave), u the smallest that gives at most g splits in all.  A ragged
+ * batch cut to its longest session's split count leaves most blocks of the
+ * short sessions empty and the others long: eight sessions of 256 .. 4096
+ * tokens ran 192 working blocks of up to 8 rounds (43 us); in splits of 3
+ * rounds over up to 512 blocks they take 23, most of it the K/V stream and
+ * the 6 us prologue.  Returns u; cnt: the splits of the lane's segment, end:
+ * of it and those before. */
+static __device__ __forceinline__ int wave_sum_i(int v) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+    return __builtin_amdgcn_readfirstlane(v);
+}
+static __device__ __forceinline__ int balance(int span, bool live, int max_span, int g, int* cnt,
+                                              int* end) {
+    const int lane = threadIdx.x & 63;
+    const int r = live ? max(1, (min(span, max_span) + AT_ROUND - 1) / AT_ROUND) : 0;
+    int u = max(1, (wave_sum_i(r) + g - 1) / g), c;
+    for (;; u++) { /* ends: with u = max r every segment has one split, and n_seg <= g */
+        c = (r + u - 1) / u;
+        if (wave_sum_i(c) <= g) break;
+    }
+    int p = c;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int t = __shfl_up(p, off, 64);
+        if (lane >= off) p += t;
+    }
+    *cnt = c;
+    *end = p;
+    return u;
+}
+
 template <int MQT, int W, int MODE>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void k_attn(AttnArgs a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int lin = (int)blockIdx.x;
-    const int total = a.nseg * a.kvh_n * a.nsplit;
-    /* chunk x of the numbering (the first total % 8 chunks one block
-     * longer) goes to XCD x; bijective for lin < total */
-    const int q = total >> 3, r = total & 7, xcd = lin & 7, j = lin >> 3;
-    const int b = xcd < r ? xcd * (q + 1) + j : r * (q + 1) + (xcd - r) * q + j;
-    const int seg = b % a.nseg, rest = b / a.nseg;
+    int seg, kvh, sp;
+    if (MODE == AM_PLAN && a.bal) {
+        /* block j of kv head x on XCD x (kvh_n is 8) */
+        const int j = lin >> 3, lane = threadIdx.x & 63;
+        const bool live = lane < a.nseg;
+        int cnt, end;
+        const int u = balance(live ? a.segs[lane].span : 0, live, a.max_span, a.bal, &cnt, &end);
+        seg = __popcll(__ballot(live && end <= j)); /* uniform */
+        if (seg >= a.nseg) return;
+        kvh = lin & 7;
+        sp = j - __builtin_amdgcn_readlane(end - cnt, seg);
+        a.split_pos = u * AT_ROUND;
+    } else {
+        /* chunk x of the numbering (the first total % 8 chunks one block
+         * longer) goes to XCD x; bijective for lin < total */
+        const int total = a.nseg * a.kvh_n * a.nsplit;
+        const int q = total >> 3, r = total & 7, xcd = lin & 7, j = lin >> 3;
+        const int b = xcd < r ? xcd * (q + 1) + j : r * (q + 1) + (xcd - r) * q + j;
+        const int rest = b / a.nseg;
+        seg = b % a.nseg;
+        kvh = rest % a.kvh_n;
+        sp = rest / a.kvh_n;
+    }
 #ifdef S2P_DIAG
-    a.probe = b < 4096 ? g_at_probe : nullptr;
+    a.probe = (sp * a.kvh_n + kvh) * a.nseg + seg < 4096 ? g_at_probe : nullptr;
 #endif
-    attn_block<MQT, W, false, MODE>(a, seg, rest % a.kvh_n, rest / a.kvh_n,
-                                    (LDS(unsigned char)*)smem_raw);
+    attn_block<MQT, W, false, MODE>(a, seg, kvh, sp, (LDS(unsigned char)*)smem_raw);
 }
 
 /* merge split partials (one thread per output element) */
@@ -80,6 +136,24 @@ __global__ __launch_bounds__(128) void k_attn_combine(const float* __restrict__ 
                                                       int qh, int nsplit) {
     /* the partials come from the previous launch: plain (cached) loads */
     attn_merge_one<false>(part, out, rows, qh, nsplit, blockIdx.x, blockIdx.y, threadIdx.x);
+}
+
+/* the same over balanced splits: a row merges its segment's count */
+__global__ __launch_bounds__(128) void k_attn_combine_bal(const float* __restrict__ part,
+                                                          uint16_t* __restrict__ out, int rows,
+                                                          int qh, int nsplit,
+                                                          const S2pAttnSeg* __restrict__ segs,
+                                                          int nseg, int max_span, int g) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x;
+    const bool live = lane < nseg;
+    S2pAttnSeg s = {};
+    if (live) s = segs[lane];
+    int cnt, end;
+    balance(s.span, live, max_span, g, &cnt, &end);
+    const uint64_t mine = __ballot(live && row >= s.row0 && row < s.row0 + s.nrows);
+    if (!mine) return; /* a row of no segment */
+    const int n = __builtin_amdgcn_readlane(cnt, __builtin_ctzll(mine));
+    attn_merge_one<false>(part, out, rows, qh, n, blockIdx.x, blockIdx.y, threadIdx.x, nsplit);
 }
 
 /* ---- tree segments: one block per (session, kv head, split) ----
@@ -123,7 +197,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nthr = (int)blockDim.x;
     const int qq = lane >> 4, c = lane & 15;
-    const SegInfo S = resolve<AM_PLAN>(a, seg, kvh);
+    const SegInfo S = resolve<AM_PLAN, 32>(a, seg, kvh);
     /* this lane's query vector: waves 0..3 rows c of head 4 kvh + wave;
      * wave 4 + e rows 16 + 4 e + c / 4 of head 4 kvh + c % 4 */
     const int r = wave < 4 ? c : 16 + 4 * (wave - 4) + (c >> 2);
@@ -335,8 +409,7 @@ static void attn_launch(const AttnArgs& a, dim3 grid, hipStream_t st) {
 
 template <int MQT, int W>
 static void attn_launch_mode(const AttnArgs& a, dim3 grid, hipStream_t st) {
-    if (a.mode == AM_CONTIG) attn_launch<MQT, W, AM_CONTIG>(a, grid, st);
-    else if (a.mode == AM_PTRS) attn_launch<MQT, W, AM_PTRS>(a, grid, st);
+    if (a.mode == AM_PTRS) attn_launch<MQT, W, AM_PTRS>(a, grid, st);
     else attn_launch<MQT, W, AM_PLAN>(a, grid, st);
 }
 
@@ -354,6 +427,21 @@ static hipError_t attn_run(AttnArgs a, int n_seg, int max_nrows, int max_span,
         }
     } else {
         tpw = tiles > 0 ? tiles : 1;
+    }
+    if (a.mode == AM_PLAN && a.part && !a.counters && a.kvh_n == 8 && n_seg <= AT_BAL_SEGS &&
+        tiles > 1 && part_floats(a.rows, a.qh, tiles) <= part_cap) {
+        a.bal = AT_MAX_BLOCKS / 8;
+        a.max_span = max_span;
+        a.nsplit = tiles; /* the partials' stride */
+        a.nseg = n_seg;
+        const dim3 grid(AT_MAX_BLOCKS);
+        if (max_nrows <= 4) attn_launch_mode<1, W>(a, grid, st);
+        else attn_launch_mode<2, W>(a, grid, st);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_attn_combine_bal, dim3(a.rows, a.qh), dim3(AT_HD), 0, st, a.part,
+                           a.out, a.rows, a.qh, a.nsplit, a.segs, n_seg, max_span, a.bal);
+        return hipGetLastError();
     }
     a.split_pos = tpw * AT_TILE * W;
     a.nsplit = (max_span + a.split_pos - 1) / a.split_pos;
@@ -387,8 +475,19 @@ extern "C" hipError_t s2pk_attention(const s2p_bf16* q, const s2p_bf16* k_cache,
     a.vc = (const uint16_t*)v_cache;
     a.pos0 = pos;
     a.max_seq = max_seq;
-    const int n_seg = (rows + AT_SEG_ROWS - 1) / AT_SEG_ROWS;
-    return attn_run(a, n_seg, rows < AT_SEG_ROWS ? rows : AT_SEG_ROWS, pos + rows, 0, st);
+    /* No scratch, so no position splits: a workgroup's waves divide a segment's
+     * positions.  Segments of four rows (one MFMA tile of query vectors) while
+     * they give at most a workgroup a CU, else of eight: a chunk of 128 rows at
+     * position 1787 takes 22 us in 256 workgroups of 8 waves, 32 in 128
+     * workgroups of 4 waves and eight rows. */
+    a.nsplit = 1;
+    a.split_pos = max_seq; /* the whole cache: one split */
+    const bool four = (int64_t)((rows + 3) / 4) * kv_heads <= s2p_cu_count();
+    a.nseg = four ? (rows + 3) / 4 : (rows + 7) / 8;
+    const dim3 grid((unsigned)(a.nseg * kv_heads));
+    if (four) attn_launch<1, 8, AM_CONTIG>(a, grid, st);
+    else attn_launch<2, 8, AM_CONTIG>(a, grid, st);
+    return hipGetLastError();
 }
 
 extern "C" hipError_t s2pk_attention_ptrs(const s2p_bf16* q, const s2p_bf16* const* k_caches,
@@ -444,12 +543,13 @@ extern "C" int64_t s2p_attn_plan_part_floats(int rows, int max_span) {
 
 extern "C" hipError_t s2p_attn_plan_fused_launch(void* q, void* out, const S2pRowPlan* plan,
                                                  const S2pAttnSeg* segs, int n_seg, int rows,
-                                                 int layer, int max_span, float* part,
-                                                 const void* qkv, const void* qn_w,
+                                                 int max_nrows, int layer, int max_span,
+                                                 float* part, const void* qkv, const void* qn_w,
                                                  const void* kn_w, const float* rope_tab,
                                                  float eps, unsigned* counters, hipStream_t st) {
     if (rows <= 0) return hipSuccess;
     if (!qkv || !rope_tab || (!qn_w) != (!kn_w)) return hipErrorInvalidValue; /* both or no norm */
+    if (max_nrows < 1 || max_nrows > AT_SEG_ROWS) return hipErrorInvalidValue;
     AttnArgs a = {};
     a.mode = AM_PLAN;
     a.q = (const uint16_t*)q;
@@ -467,7 +567,7 @@ extern "C" hipError_t s2p_attn_plan_fused_launch(void* q, void* out, const S2pRo
     a.kn_w = (const uint16_t*)kn_w;
     a.rope_tab = rope_tab;
     a.eps = eps;
-    return attn_run(a, n_seg, AT_SEG_ROWS, max_span, s2p_attn_plan_part_floats(rows, max_span),
+    return attn_run(a, n_seg, max_nrows, max_span, s2p_attn_plan_part_floats(rows, max_span),
                     st);
 }
 

@@ -75,6 +75,7 @@ struct AttnArgs {
     const uint16_t* kn_w;
     const float* rope_tab; /* [rows][64][cos, sin] of the plan's positions */
     float eps;
+    int bal, max_span; /* PLAN: blocks a kv head for balanced splits, or 0 */
 };
 
 struct SegInfo {
@@ -86,14 +87,14 @@ struct SegInfo {
 
 /* MODE is a compile-time constant: each caller kind gets its own kernel,
  * with no run-time branch over the modes */
-template <int MODE>
+template <int MODE, int SR>
 S2P_DEV SegInfo resolve(const AttnArgs& a, int seg, int kvh) {
     SegInfo s;
     s.vis = nullptr;
     s.first = 0;
     if constexpr (MODE == AM_CONTIG) {
-        s.row0 = seg * AT_SEG_ROWS;
-        s.nrows = min(AT_SEG_ROWS, a.rows - s.row0);
+        s.row0 = seg * SR;
+        s.nrows = min(SR, a.rows - s.row0);
         s.L = a.pos0 + s.row0;
         s.span = min(s.L + s.nrows, a.max_seq); /* never read past the cache */
         s.kp = a.kc + (size_t)kvh * a.max_seq * AT_HD;
@@ -197,9 +198,10 @@ S2P_DEV float ld_f(const float* p) {
 
 template <bool COH = true>
 S2P_DEV void attn_merge_one(const float* part, uint16_t* out, int rows, int qh, int nsplit,
-                            int row, int h, int d) {
-    const size_t p0 = ((size_t)row * qh + h) * nsplit;
-    const float* po = part + (size_t)rows * qh * nsplit * 2;
+                            int row, int h, int d, int stride = 0) {
+    if (!stride) stride = nsplit; /* splits the layout holds per (row, head) */
+    const size_t p0 = ((size_t)row * qh + h) * stride;
+    const float* po = part + (size_t)rows * qh * stride * 2;
     float M = -INFINITY;
     for (int s = 0; s < nsplit; s++) M = fmaxf(M, ld_f<COH>(part + (p0 + s) * 2));
     const float Ms = M == -INFINITY ? 0.f : M;
@@ -249,7 +251,7 @@ __device__ bool attn_block(const AttnArgs& a, int seg, int kvh, int sp, LDS(unsi
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int qq = lane >> 4, c = lane & 15;
-    const SegInfo S = resolve<MODE>(a, seg, kvh);
+    const SegInfo S = resolve<MODE, 4 * MQT>(a, seg, kvh);
     /* the mask words of this lane's query rows 4 qt + c / 4 (query vector
      * 16 qt + c), loaded once and first (every later load is then younger,
      * so the tile loop's waits can count the prefetches in flight) */

@@ -371,7 +371,7 @@ static s2p_status draft_step_at(s2p_draft_model* m, s2p_draft_state* s, const vo
                    ssq_a, GEMV_EPI_STORE, NULL, st));
     /* qk-norm, RoPE, K/V append at slot pos and attention over [0, pos]
      * (the normed q rows land in xcat, no longer needed) */
-    HIPTRY(s2p_attn_plan_fused_launch(m->xcat.data, m->attn.data, &plan, seg, 1, 1, 0, span_max,
+    HIPTRY(s2p_attn_plan_fused_launch(m->xcat.data, m->attn.data, &plan, seg, 1, 1, 1, 0, span_max,
                                       (float*)(ws + WS_PART), m->qkv.data, m->q_norm.data,
                                       m->k_norm.data, (const float*)(ws + WS_ROPE), D_EPS,
                                       (unsigned*)(ws + WS_CTR), st));

@@ -311,7 +311,7 @@ static s2p_status run_layers(s2pfa* f, int B, int p, hipStream_t st) {
         const s2pfa_layer* L = &f->w.layers[l];
         TRY(gemv(&L->wqkv, B, f->x, f->qkv, FA_QKV, GEMV_X_NORM, L->attn_norm.data, f->ssq_a,
                  GEMV_EPI_STORE, NULL, st));
-        HIPCHK(s2p_attn_plan_fused_launch(f->q, f->attn, &pl, seg, B, B, l, p + 1, f->part, f->qkv,
+        HIPCHK(s2p_attn_plan_fused_launch(f->q, f->attn, &pl, seg, B, B, 1, l, p + 1, f->part, f->qkv,
                                           NULL, NULL, rope, FA_EPS, f->counters, st));
         TRY(gemv(&L->wo, B, f->attn, f->x, FA_DIM, GEMV_X_PLAIN, NULL, NULL, GEMV_EPI_RESID,
                  f->ssq_b, st));

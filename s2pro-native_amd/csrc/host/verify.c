@@ -691,8 +691,9 @@ s2p_status s2p_verify_forward(s2p_backbone* b, const void* x_in, void* logits, h
                                                 l, b->max_span, b->attn_part, b->attn_part_floats, st),
                            "tree attention"));
         } else
-        S2P_TRY(hip_ok(s2p_attn_plan_fused_launch(b->q, b->attn, &plan, b->d_segs, b->n_seg, M, l,
-                                                  b->max_span, b->attn_part, b->qkv,
+        S2P_TRY(hip_ok(s2p_attn_plan_fused_launch(b->q, b->attn, &plan, b->d_segs, b->n_seg, M,
+                                                  b->R < 8 ? b->R : 8, l, b->max_span,
+                                                  b->attn_part, b->qkv,
                                                   L->q_norm.data, L->k_norm.data, b->d_rope,
                                                   NORM_EPS, NULL, st),
                        "attention"));

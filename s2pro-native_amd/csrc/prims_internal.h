@@ -92,7 +92,7 @@ hipError_t s2p_attn_plan_launch(const void* q, void* out, const S2pRowPlan* plan
                                 const S2pAttnSeg* segs, int n_seg, int rows, int layer,
                                 int max_span, float* part, hipStream_t st);
 /* The same, fused with qk-norm + RoPE + KV append (q is the scratch the q
- * rows are written to) and, with counters ([n_seg * 8], zero between calls),
+ * rows are written to; no segment has more than max_nrows <= 8 rows) and, with counters ([n_seg * 8], zero between calls),
  * with the split merge done by the last split of each block. */
 /* qn_w = kn_w = NULL: RoPE without qk-norm (a model without qk-norm) */
 /* Tree attention over bf16 caches (csrc/attention.hip): segs [n_seg] hold
@@ -104,8 +104,8 @@ hipError_t s2p_attn_tree_launch(const void* q, void* out, const S2pRowPlan* plan
                                 int layer, int max_span, float* part, int64_t part_cap,
                                 hipStream_t st);
 hipError_t s2p_attn_plan_fused_launch(void* q, void* out, const S2pRowPlan* plan,
-                                      const S2pAttnSeg* segs, int n_seg, int rows, int layer,
-                                      int max_span, float* part, const void* qkv,
+                                      const S2pAttnSeg* segs, int n_seg, int rows, int max_nrows,
+                                      int layer, int max_span, float* part, const void* qkv,
                                       const void* qn_w, const void* kn_w, const float* rope_tab,
                                       float eps, unsigned* counters, hipStream_t st);
 int64_t    s2p_attn_plan_part_floats(int rows, int max_span);

@@ -244,3 +244,58 @@ def test_attention_decode_edges(lib, bw, lens):
             # one bf16 rounding (2^-9) of an f32 sum, f32 exponentials
             bound = 2.0 ** -8 * np.abs(want) + 2e-4 * np.abs(vs[i][h // 4, :L]).max()
             assert (np.abs(got[i, h] - want) <= bound).all(), (bw, L, h)
+
+
+# four- and eight-row segments (128 rows fill the 256 workgroups of four), a
+# wave's round (256 positions) and its edges
+@pytest.mark.parametrize("rows,pos,max_seq", [(3, 0, 3), (4, 252, 256), (7, 250, 300),
+                                              (128, 129, 257), (129, 5, 160)])
+def test_attention_contig_segments(lib, rows, pos, max_seq):
+    kc, vc = cache(rows + pos, max_seq)
+    q = bf16_bits(np.random.default_rng(pos).standard_normal((rows, 4096)).astype(np.float32))
+    out = empty((rows, 4096))
+    s2pamd.hip_check(lib.s2pk_attention(P(to_dev(q)), P(to_dev(kc)), P(to_dev(vc)), P(out), rows,
+                                        32, 8, 128, pos, max_seq, S()))
+    got = bf16_vals(to_host(out, np.uint16))
+    for r0 in range(0, rows, 32):  # the oracle holds a position's 64 newest rows
+        n = min(32, rows - r0)
+        exact = po.attention_f64(q[r0:r0 + n], kc, vc, n, 32, 8, 128, pos + r0, max_seq)
+        assert np.abs(got[r0:r0 + n] - exact).max() < 2e-2, r0
+
+
+# ragged sessions: fewer rounds of 128 positions than blocks and more, one
+# session alone, the most sessions that share the blocks by length and one more
+@pytest.mark.parametrize("R,Ls", [(5, [1, 2000, 127, 128, 640]), (3, [4100]), (8, [9000, 1, 500]),
+                                  (5, [40 * i + 1 for i in range(32)]),
+                                  (4, [7 * i for i in range(33)])])
+def test_attention_plan_ragged(lib, R, Ls):
+    import ctypes
+    n = len(Ls)
+    rng = np.random.default_rng(R + n)
+    cap = max(Ls) + R
+    q = bf16_bits(rng.standard_normal((n * R, 4096)).astype(np.float32) * 2)
+    kvs = [bf16_bits(rng.standard_normal((16, cap, 128)).astype(np.float32)) for _ in Ls]
+    kvd = [to_dev(k) for k in kvs]
+    kvp = to_dev(np.array([k.data_ptr() for k in kvd], np.int64))
+    posd = to_dev(np.concatenate([np.arange(L, L + R, dtype=np.int32) for L in Ls]))
+    sessd = to_dev(np.repeat(np.arange(n, dtype=np.int32), R))
+    plan = RowPlan(posd.data_ptr(), posd.data_ptr(), sessd.data_ptr(), None, kvp.data_ptr(), None,
+                   16 * cap * 128, cap)
+    segs = (AttnSeg * n)(*[AttnSeg(i, L, i * R, R, L + R, i * R, kvd[i].data_ptr())
+                           for i, L in enumerate(Ls)])
+    segd = to_dev(np.frombuffer(bytes(segs), np.uint8).copy())
+    part = empty((lib.s2pk_attention_part_floats(n * R, 32, cap),), dtype=torch.float32)
+    part.fill_(float("nan"))  # what no block writes is not read
+    out = empty((n * R, 4096))
+    fn = lib.s2p_attn_plan_launch
+    fn.restype = ctypes.c_int
+    fn.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
+                                           ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
+                                           ctypes.c_void_p]
+    s2pamd.hip_check(fn(P(to_dev(q)), P(out), ctypes.byref(plan), P(segd), n, n * R, 0, cap,
+                        P(part), S()))
+    got = bf16_vals(to_host(out, np.uint16))
+    for i, L in enumerate(Ls):
+        exact = po.attention_f64(q[i * R:(i + 1) * R], np.ascontiguousarray(kvs[i][:8]),
+                                 np.ascontiguousarray(kvs[i][8:]), R, 32, 8, 128, L, cap)
+        assert np.abs(got[i * R:(i + 1) * R] - exact).max() < 2e-2, (i, L)
