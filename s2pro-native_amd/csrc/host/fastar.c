@@ -1,12 +1,10 @@
 /* s2pro MI355X — the fast-AR residual-codebook decoder (include/s2pro/fastar.h).
  *
  * The reference loop (src/fastar/fastar.cu:726-789) on the verify engine:
- * every row b of a frame batch is a one-row attention segment over its own
- * depth-11 cache (per row [4 layers][16 planes][11][128] bf16, the verify
- * path's cache layout), so RoPE + K/V append + attention of all rows is one
- * plan-mode launch per layer with qk-norm off.  The plans of positions 0..9
- * (row positions, slots, visibility, segments, RoPE rows) are written once at
- * creation.  Per layer: wqkv with the attention RMSNorm in its staging; the
+ * every row b of a frame batch has its own depth-11 cache (per row [4
+ * layers][16 planes][11][128] bf16, the verify path's cache layout); RoPE, K/V
+ * append and attention of all rows is one launch per layer (fa_attn.hip) over
+ * the RoPE rows of positions 0..9, computed once at creation.  Per layer: wqkv with the attention RMSNorm in its staging; the
  * attention; wo with the residual add (and the sums of squares of the new
  * residual) in its epilogue; w13 with the FFN RMSNorm in its staging and
  * SwiGLU in its epilogue; w2 with the residual add.  The step input and the
@@ -45,20 +43,12 @@ struct s2pfa {
     int owns;
     int max_b;
     /* device workspace for max_b rows */
-    uint16_t *x, *qkv, *q, *attn, *ffn, *logits;
-    float *ssq_a, *ssq_b, *part;
-    unsigned* counters;
+    uint16_t *x, *qkv, *attn, *ffn, *logits;
+    float *ssq_a, *ssq_b;
     int32_t* stage;   /* [9][max_b] */
     int32_t* sem_dev; /* [max_b] (host-pointer entry point) */
     uint16_t* kv;     /* [max_b][FA_ROWKV] */
-    /* per position p: the plan arrays, segments and RoPE rows */
-    int32_t* d_pos;   /* [FA_NPOS][max_b]: p */
-    int32_t* d_slot;  /* [FA_NPOS][max_b]: p */
-    int32_t* d_sess;  /* [max_b]: b */
-    uint64_t* d_vis;  /* [max_b]: 1 */
-    void** d_kv;      /* [max_b]: row b's cache */
-    S2pAttnSeg* d_seg; /* [FA_NPOS][max_b] */
-    float* d_rope;    /* [FA_NPOS][max_b][64][2] */
+    float* d_rope;    /* [FA_NPOS][64][2]: the RoPE row of each position */
     int32_t* codes_dev; /* host-codes VQ entry point, grown on demand */
     int codes_cap;
     int32_t* stage_host;
@@ -87,92 +77,36 @@ static s2p_status dalloc(void* pp, size_t bytes) {
     return S2P_OK;
 }
 
-static S2pRowPlan plan_of(const s2pfa* f, int p) {
-    S2pRowPlan pl;
-    memset(&pl, 0, sizeof(pl));
-    pl.pos = f->d_pos + (size_t)p * f->max_b;
-    pl.slot = f->d_slot + (size_t)p * f->max_b;
-    pl.sess = f->d_sess;
-    pl.vis = f->d_vis;
-    pl.kv = (void* const*)f->d_kv;
-    pl.kvs = NULL;
-    pl.layer_stride = FA_LSTRIDE;
-    pl.max_seq = S2P_FA_SEQ;
-    return pl;
-}
-
-/* workspace and the per-position plans (host tables uploaded once) */
+/* workspace and the positions' RoPE rows */
 static s2p_status build(s2pfa* f, hipStream_t st) {
-    const int B = f->max_b, NP = FA_NPOS;
+    const int B = f->max_b;
     TRY(dalloc(&f->x, (size_t)B * FA_DIM * 2));
     TRY(dalloc(&f->qkv, (size_t)B * FA_QKV * 2));
-    TRY(dalloc(&f->q, (size_t)B * FA_Q * 2));
     TRY(dalloc(&f->attn, (size_t)B * FA_Q * 2));
     TRY(dalloc(&f->ffn, (size_t)B * FA_FFN * 2));
     TRY(dalloc(&f->logits, (size_t)B * S2P_FA_CB * 2));
     TRY(dalloc(&f->ssq_a, (size_t)(FA_DIM / GEMV_SSQ_COLS) * GEMV_MAX_M * 4));
     TRY(dalloc(&f->ssq_b, (size_t)(FA_DIM / GEMV_SSQ_COLS) * GEMV_MAX_M * 4));
-    TRY(dalloc(&f->part, (size_t)s2p_attn_plan_part_floats(B, S2P_FA_SEQ) * 4));
-    TRY(dalloc(&f->counters, (size_t)B * 8 * 4));
     TRY(dalloc(&f->stage, (size_t)(S2P_FA_NCB - 1) * B * 4));
     TRY(dalloc(&f->sem_dev, (size_t)B * 4));
     TRY(dalloc(&f->kv, (size_t)B * FA_ROWKV * 2));
-    TRY(dalloc(&f->d_pos, (size_t)NP * B * 4));
-    TRY(dalloc(&f->d_slot, (size_t)NP * B * 4));
-    TRY(dalloc(&f->d_sess, (size_t)B * 4));
-    TRY(dalloc(&f->d_vis, (size_t)B * 8));
-    TRY(dalloc(&f->d_kv, (size_t)B * sizeof(void*)));
-    TRY(dalloc(&f->d_seg, (size_t)NP * B * sizeof(S2pAttnSeg)));
-    TRY(dalloc(&f->d_rope, (size_t)NP * B * 128 * 4));
+    TRY(dalloc(&f->d_rope, (size_t)FA_NPOS * 128 * 4));
     if (hipHostMalloc((void**)&f->stage_host, (size_t)(S2P_FA_NCB - 1) * B * 4, 0) != hipSuccess) {
         f->stage_host = NULL;
         return S2P_ERR_OOM;
     }
-    int32_t* pos = (int32_t*)malloc((size_t)NP * B * 4);
-    int32_t* sess = (int32_t*)malloc((size_t)B * 4);
-    uint64_t* vis = (uint64_t*)malloc((size_t)B * 8);
-    void** kv = (void**)malloc((size_t)B * sizeof(void*));
-    S2pAttnSeg* seg = (S2pAttnSeg*)malloc((size_t)NP * B * sizeof(S2pAttnSeg));
-    s2p_status rc = pos && sess && vis && kv && seg ? S2P_OK : S2P_ERR_OOM;
-    if (rc == S2P_OK) {
-        for (int b = 0; b < B; b++) {
-            sess[b] = b;
-            vis[b] = 1ull; /* a row sees its own slot and the prefix before it */
-            kv[b] = f->kv + (size_t)b * FA_ROWKV;
-        }
-        for (int p = 0; p < NP; p++)
-            for (int b = 0; b < B; b++) {
-                pos[p * B + b] = p;
-                S2pAttnSeg* g = &seg[p * B + b];
-                g->sess = b;
-                g->L = p;
-                g->row0 = b;
-                g->nrows = 1;
-                g->span = p + 1;
-                g->first = b;
-                g->kv = kv[b];
-            }
-        if (hipMemcpy(f->d_pos, pos, (size_t)NP * B * 4, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(f->d_slot, pos, (size_t)NP * B * 4, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(f->d_sess, sess, (size_t)B * 4, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(f->d_vis, vis, (size_t)B * 8, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(f->d_kv, kv, (size_t)B * sizeof(void*), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(f->d_seg, seg, (size_t)NP * B * sizeof(S2pAttnSeg), hipMemcpyHostToDevice) !=
-                hipSuccess ||
-            hipMemset(f->counters, 0, (size_t)B * 8 * 4) != hipSuccess)
-            rc = S2P_ERR_CUDA;
-    }
-    free(pos);
-    free(sess);
-    free(vis);
-    free(kv);
-    free(seg);
-    if (rc != S2P_OK) return rc;
-    for (int p = 0; p < NP; p++) {
-        const S2pRowPlan pl = plan_of(f, p);
-        HIPCHK(s2p_rope_tab_launch(&pl, B, FA_ROPE_BASE, f->d_rope + (size_t)p * B * 128, st));
-    }
-    HIPCHK(hipStreamSynchronize(st));
+    int32_t pos[FA_NPOS];
+    for (int p = 0; p < FA_NPOS; p++) pos[p] = p;
+    int32_t* d_pos = NULL;
+    TRY(dalloc(&d_pos, sizeof(pos)));
+    S2pRowPlan pl;
+    memset(&pl, 0, sizeof(pl));
+    pl.pos = d_pos;
+    hipError_t e = hipMemcpy(d_pos, pos, sizeof(pos), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = s2p_rope_tab_launch(&pl, FA_NPOS, FA_ROPE_BASE, f->d_rope, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    (void)hipFree(d_pos);
+    HIPCHK(e);
     return S2P_OK;
 }
 
@@ -255,10 +189,8 @@ s2p_status s2pfa_create_random(s2pfa** out, s2p_weight_q quant, int max_b, uint6
 
 void s2pfa_free(s2pfa* f) {
     if (!f) return;
-    void* ps[] = {f->x,     f->qkv,    f->q,     f->attn,   f->ffn,  f->logits,
-                  f->ssq_a, f->ssq_b,  f->part,  f->counters, f->stage, f->sem_dev,
-                  f->kv,    f->d_pos,  f->d_slot, f->d_sess, f->d_vis, f->d_kv,
-                  f->d_seg, f->d_rope, f->codes_dev};
+    void* ps[] = {f->x,     f->qkv,   f->attn,    f->ffn, f->logits, f->ssq_a,
+                  f->ssq_b, f->stage, f->sem_dev, f->kv,  f->d_rope, f->codes_dev};
     for (size_t i = 0; i < sizeof(ps) / sizeof(ps[0]); i++)
         if (ps[i]) (void)hipFree(ps[i]);
     if (f->stage_host) (void)hipHostFree(f->stage_host);
@@ -304,15 +236,12 @@ static s2p_status gemv(const s2p_linear* lin, int M, const void* x, void* y, int
 
 /* the 4 layers on x (sums of squares in ssq_a) at position p, K/V at slot p */
 static s2p_status run_layers(s2pfa* f, int B, int p, hipStream_t st) {
-    const S2pRowPlan pl = plan_of(f, p);
-    const S2pAttnSeg* seg = f->d_seg + (size_t)p * f->max_b;
-    const float* rope = f->d_rope + (size_t)p * f->max_b * 128;
     for (int l = 0; l < S2P_FA_LAYERS; l++) {
         const s2pfa_layer* L = &f->w.layers[l];
         TRY(gemv(&L->wqkv, B, f->x, f->qkv, FA_QKV, GEMV_X_NORM, L->attn_norm.data, f->ssq_a,
                  GEMV_EPI_STORE, NULL, st));
-        HIPCHK(s2p_attn_plan_fused_launch(f->q, f->attn, &pl, seg, B, B, 1, l, p + 1, f->part, f->qkv,
-                                          NULL, NULL, rope, FA_EPS, f->counters, st));
+        HIPCHK(s2p_fa_attn_launch(f->qkv, f->d_rope, 128, f->kv + l * FA_LSTRIDE, FA_ROWKV, f->attn,
+                                  B, p, 1, st));
         TRY(gemv(&L->wo, B, f->attn, f->x, FA_DIM, GEMV_X_PLAIN, NULL, NULL, GEMV_EPI_RESID,
                  f->ssq_b, st));
         TRY(gemv(&L->w13, B, f->x, f->ffn, FA_FFN, GEMV_X_NORM, L->ffn_norm.data, f->ssq_b,

@@ -64,6 +64,13 @@ hipError_t s2p_qkrope_append_launch(const void* qkv, void* q_out, const void* qn
  * ([width/16][128]); the 10-codebook VQ embedding added onto rows. */
 hipError_t s2p_fa_embed_ssq_launch(const void* table, const int32_t* ids, int n_ids, void* x,
                                    float* ssq, int rows, int width, hipStream_t st);
+/* Fast-AR attention (csrc/fa_attn.hip): RoPE, K/V append and attention of the
+ * rows s * nn .. + nn - 1 of every session s at positions p0 .. p0 + nn - 1
+ * (nn 1 or 2); rope: the (cos, sin) row of position p at p * rope_stride; kv:
+ * one layer of session 0, the sessions sess_stride elements apart. */
+hipError_t s2p_fa_attn_launch(const void* qkv, const float* rope, int rope_stride, void* kv,
+                              int64_t sess_stride, void* out, int n_sess, int p0, int nn,
+                              hipStream_t st);
 hipError_t s2p_fa_vq_embed_add_launch(const void* table, const int32_t* codes, int T, void* rows,
                                       int dim, hipStream_t st);
 /* Draft step prologue: the one-row plan (pos/slot/sess/vis/kv arrays behind

@@ -300,3 +300,61 @@ def test_frame_rows_past_eight(lib, decoder):
     finally:
         sync()
         lib.s2pfa_free(big)
+
+
+# no earlier slot, one, all ten; one new row a session and two
+@pytest.mark.parametrize("n,p0,nn", [(1, 0, 1), (3, 1, 1), (2, 10, 1), (3, 0, 2), (2, 9, 2)])
+def test_fa_attention(lib, n, p0, nn):
+    import ctypes
+    r = np.random.default_rng(100 * n + 10 * p0 + nn)
+    rows = n * nn
+    qkv = bf16_bits(r.standard_normal((rows, 6144)).astype(np.float32))
+    kv = bf16_bits(r.standard_normal((n, 16, 11, 128)).astype(np.float32))
+    ang = np.outer(np.arange(11), r.uniform(0.01, 1.0, 64))
+    rope = np.stack([np.cos(ang), np.sin(ang)], -1).astype(np.float32)
+    kvd, out = to_dev(kv), empty((rows, 4096))
+    fn = lib.s2p_fa_attn_launch
+    fn.restype = ctypes.c_int
+    fn.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64,
+                   ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    s2pamd.hip_check(fn(P(to_dev(qkv)), P(to_dev(rope)), 128, P(kvd), 16 * 11 * 128, P(out), n, p0,
+                        nn, S()), "fa_attn")
+
+    def roped(v, p):  # interleaved pairs, rounded to bf16
+        v = v.astype(np.float32).reshape(-1, 64, 2)
+        c, s_ = rope[p, :, 0], rope[p, :, 1]
+        o = np.stack([v[..., 0] * c - v[..., 1] * s_, v[..., 0] * s_ + v[..., 1] * c], -1)
+        return bf16_vals(bf16_bits(o.reshape(-1, 128)))
+
+    got = bf16_vals(to_host(out, np.uint16)).reshape(rows, 32, 128).astype(np.float64)
+    after = bf16_vals(to_host(kvd, np.uint16)).reshape(n, 16, 11, 128)
+    x = bf16_vals(qkv)
+    want_kv = bf16_vals(kv).copy()
+    for s in range(n):
+        for i in range(nn):
+            row, p = s * nn + i, p0 + i
+            want_kv[s, :8, p] = roped(x[row, 4096:5120], p)
+            want_kv[s, 8:, p] = x[row, 5120:].reshape(8, 128)
+            q = roped(x[row, :4096], p).astype(np.float64)
+            for h in range(32):
+                k = want_kv[s, h // 4, :p + 1].astype(np.float64)
+                v = want_kv[s, 8 + h // 4, :p + 1].astype(np.float64)
+                sc = k @ q[h] / np.sqrt(128.0)
+                w = np.exp(sc - sc.max())
+                want = (w / w.sum()) @ v
+                # one bf16 rounding (2^-9); a key or query element on a rounding
+                # tie may fall the other way (2^-8 of one product in 128)
+                bound = 2.0 ** -8 * np.abs(want) + 2e-3 * np.abs(v).max()
+                assert (np.abs(got[row, h] - want) <= bound).all(), (row, h)
+    assert np.abs(after - want_kv).max() <= 2.0 ** -7 * np.abs(want_kv).max()
+
+
+@pytest.mark.parametrize("V,off", [(8, 0), (4096, 3), (4099, 0), (20000, 0)])
+def test_argmax_layouts(lib, V, off):
+    """16-byte pieces and the rest (an odd width, an odd address)."""
+    r = np.random.default_rng(V)
+    bits = bf16_bits(r.standard_normal((3, V)).astype(np.float32).round(1))
+    d = to_dev(np.concatenate([np.zeros(off, np.uint16), bits.ravel()]))[off:]
+    ids = empty((3,), torch.int32)
+    assert lib.s2pk_argmax(P(d), P(ids), 3, V, S()) == 0
+    assert np.array_equal(to_host(ids), bf16_vals(bits).argmax(1))
