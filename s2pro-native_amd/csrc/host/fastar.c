@@ -9,8 +9,9 @@
  * residual) in its epilogue; w13 with the FFN RMSNorm in its staging and
  * SwiGLU in its epilogue; w2 with the residual add.  The step input and the
  * prime pass's hidden enter through a gather / copy that also writes the
- * sums of squares.  Launches per frame: 1 + 4 x 5 (prime) and 9 x (1 + 4 x 5
- * + head + argmax). */
+ * sums of squares.  Launches per frame of
+ * up to 8 rows: 9 x (1 + 4 x 5 + head + argmax) + 1 (the prime rows go with the
+ * first code's); above that 1 + 4 x 5 more. */
 #include "s2pro/fastar.h"
 
 #include <math.h>
@@ -37,6 +38,7 @@ unsigned* s2p_gemm_ctx_counters(void);
 #define FA_EPS 1e-6f
 #define FA_ROPE_BASE 1000000.0f
 #define FA_NPOS 10 /* positions 0 (prime) .. 9 */
+#define FA_BOTH 16 /* most rows of a pass over positions 0 and 1 together */
 
 struct s2pfa {
     s2pfa_weights w;
@@ -46,6 +48,7 @@ struct s2pfa {
     uint16_t *x, *qkv, *attn, *ffn, *logits;
     float *ssq_a, *ssq_b;
     int32_t* stage;   /* [9][max_b] */
+    int32_t* odd;     /* [FA_BOTH / 2]: 1, 3, 5, .. */
     int32_t* sem_dev; /* [max_b] (host-pointer entry point) */
     uint16_t* kv;     /* [max_b][FA_ROWKV] */
     float* d_rope;    /* [FA_NPOS][64][2]: the RoPE row of each position */
@@ -80,10 +83,13 @@ static s2p_status dalloc(void* pp, size_t bytes) {
 /* workspace and the positions' RoPE rows */
 static s2p_status build(s2pfa* f, hipStream_t st) {
     const int B = f->max_b;
-    TRY(dalloc(&f->x, (size_t)B * FA_DIM * 2));
-    TRY(dalloc(&f->qkv, (size_t)B * FA_QKV * 2));
-    TRY(dalloc(&f->attn, (size_t)B * FA_Q * 2));
-    TRY(dalloc(&f->ffn, (size_t)B * FA_FFN * 2));
+    /* rows of a pass: a frame of up to FA_BOTH / 2 sessions starts with two each */
+    const int R = 2 * B <= FA_BOTH ? 2 * B : B > FA_BOTH ? B : FA_BOTH;
+    TRY(dalloc(&f->x, (size_t)R * FA_DIM * 2));
+    TRY(dalloc(&f->qkv, (size_t)R * FA_QKV * 2));
+    TRY(dalloc(&f->attn, (size_t)R * FA_Q * 2));
+    TRY(dalloc(&f->ffn, (size_t)R * FA_FFN * 2));
+    TRY(dalloc(&f->odd, (FA_BOTH / 2) * 4));
     TRY(dalloc(&f->logits, (size_t)B * S2P_FA_CB * 2));
     TRY(dalloc(&f->ssq_a, (size_t)(FA_DIM / GEMV_SSQ_COLS) * GEMV_MAX_M * 4));
     TRY(dalloc(&f->ssq_b, (size_t)(FA_DIM / GEMV_SSQ_COLS) * GEMV_MAX_M * 4));
@@ -95,7 +101,8 @@ static s2p_status build(s2pfa* f, hipStream_t st) {
         f->stage_host = NULL;
         return S2P_ERR_OOM;
     }
-    int32_t pos[FA_NPOS];
+    int32_t pos[FA_NPOS], odd[FA_BOTH / 2];
+    for (int b = 0; b < FA_BOTH / 2; b++) odd[b] = 2 * b + 1;
     for (int p = 0; p < FA_NPOS; p++) pos[p] = p;
     int32_t* d_pos = NULL;
     TRY(dalloc(&d_pos, sizeof(pos)));
@@ -103,6 +110,7 @@ static s2p_status build(s2pfa* f, hipStream_t st) {
     memset(&pl, 0, sizeof(pl));
     pl.pos = d_pos;
     hipError_t e = hipMemcpy(d_pos, pos, sizeof(pos), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(f->odd, odd, sizeof(odd), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = s2p_rope_tab_launch(&pl, FA_NPOS, FA_ROPE_BASE, f->d_rope, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     (void)hipFree(d_pos);
@@ -190,7 +198,8 @@ s2p_status s2pfa_create_random(s2pfa** out, s2p_weight_q quant, int max_b, uint6
 void s2pfa_free(s2pfa* f) {
     if (!f) return;
     void* ps[] = {f->x,     f->qkv,   f->attn,    f->ffn, f->logits, f->ssq_a,
-                  f->ssq_b, f->stage, f->sem_dev, f->kv,  f->d_rope, f->codes_dev};
+                  f->ssq_b, f->stage, f->sem_dev, f->kv,  f->d_rope, f->codes_dev,
+                  f->odd};
     for (size_t i = 0; i < sizeof(ps) / sizeof(ps[0]); i++)
         if (ps[i]) (void)hipFree(ps[i]);
     if (f->stage_host) (void)hipHostFree(f->stage_host);
@@ -234,19 +243,21 @@ static s2p_status gemv(const s2p_linear* lin, int M, const void* x, void* y, int
     return S2P_OK;
 }
 
-/* the 4 layers on x (sums of squares in ssq_a) at position p, K/V at slot p */
-static s2p_status run_layers(s2pfa* f, int B, int p, hipStream_t st) {
+/* the 4 layers on x (sums of squares in ssq_a): nn rows a session, B * nn in
+ * all, at positions p .. p + nn - 1 */
+static s2p_status run_layers(s2pfa* f, int B, int p, int nn, hipStream_t st) {
+    const int M = B * nn;
     for (int l = 0; l < S2P_FA_LAYERS; l++) {
         const s2pfa_layer* L = &f->w.layers[l];
-        TRY(gemv(&L->wqkv, B, f->x, f->qkv, FA_QKV, GEMV_X_NORM, L->attn_norm.data, f->ssq_a,
+        TRY(gemv(&L->wqkv, M, f->x, f->qkv, FA_QKV, GEMV_X_NORM, L->attn_norm.data, f->ssq_a,
                  GEMV_EPI_STORE, NULL, st));
         HIPCHK(s2p_fa_attn_launch(f->qkv, f->d_rope, 128, f->kv + l * FA_LSTRIDE, FA_ROWKV, f->attn,
-                                  B, p, 1, st));
-        TRY(gemv(&L->wo, B, f->attn, f->x, FA_DIM, GEMV_X_PLAIN, NULL, NULL, GEMV_EPI_RESID,
+                                  B, p, nn, st));
+        TRY(gemv(&L->wo, M, f->attn, f->x, FA_DIM, GEMV_X_PLAIN, NULL, NULL, GEMV_EPI_RESID,
                  f->ssq_b, st));
-        TRY(gemv(&L->w13, B, f->x, f->ffn, FA_FFN, GEMV_X_NORM, L->ffn_norm.data, f->ssq_b,
+        TRY(gemv(&L->w13, M, f->x, f->ffn, FA_FFN, GEMV_X_NORM, L->ffn_norm.data, f->ssq_b,
                  GEMV_EPI_SWIGLU, NULL, st));
-        TRY(gemv(&L->w2, B, f->ffn, f->x, FA_DIM, GEMV_X_PLAIN, NULL, NULL, GEMV_EPI_RESID,
+        TRY(gemv(&L->w2, M, f->ffn, f->x, FA_DIM, GEMV_X_PLAIN, NULL, NULL, GEMV_EPI_RESID,
                  f->ssq_a, st));
     }
     return S2P_OK;
@@ -254,16 +265,35 @@ static s2p_status run_layers(s2pfa* f, int B, int p, hipStream_t st) {
 
 static s2p_status frame(s2pfa* f, const void* hidden, const int32_t* sem_dev, int B,
                         uint16_t* logits_all, hipStream_t st) {
-    /* prime: K/V at position 0 from the final-normed hidden; its logits are
-     * never read (the reference computes and discards them) */
-    HIPCHK(s2p_resid_init_launch(hidden, f->x, f->ssq_a, B, FA_DIM, st));
-    TRY(run_layers(f, B, 0, st));
+    /* Prime: K/V at position 0 from the final-normed hidden; its logits are
+     * never read (the reference computes and discards them).  The row of
+     * position 1, the semantic code's embedding, is known as well, so one pass
+     * over the weights takes both rows of every session, hidden then code,
+     * while they are at most the 16 rows of a GEMV. */
+    const int both = 2 * B <= FA_BOTH;
+    if (!both) {
+        HIPCHK(s2p_resid_init_launch(hidden, f->x, f->ssq_a, B, FA_DIM, st));
+        TRY(run_layers(f, B, 0, 1, st));
+    }
     for (int cb = 1; cb < S2P_FA_NCB; cb++) {
         const int32_t* ids = cb == 1 ? sem_dev : f->stage + (size_t)(cb - 2) * B;
-        HIPCHK(s2p_fa_embed_ssq_launch(f->w.emb.data, ids, S2P_FA_CB, f->x, f->ssq_a, B, FA_DIM, st));
-        TRY(run_layers(f, B, cb, st));
+        const uint16_t* x = f->x;
+        const float* ssq = f->ssq_a;
+        if (cb == 1 && both) {
+            HIPCHK(s2p_fa_prime_launch(hidden, f->w.emb.data, ids, S2P_FA_CB, f->x, f->ssq_a, B,
+                                       FA_DIM, st));
+            TRY(run_layers(f, B, 0, 2, st));
+            /* the code rows for the head (attn and ssq_b are free) */
+            HIPCHK(s2p_fa_embed_ssq_launch(f->x, f->odd, 2 * B, f->attn, f->ssq_b, B, FA_DIM, st));
+            x = f->attn;
+            ssq = f->ssq_b;
+        } else {
+            HIPCHK(s2p_fa_embed_ssq_launch(f->w.emb.data, ids, S2P_FA_CB, f->x, f->ssq_a, B, FA_DIM,
+                                           st));
+            TRY(run_layers(f, B, cb, 1, st));
+        }
         uint16_t* lg = logits_all ? logits_all + (size_t)(cb - 1) * B * S2P_FA_CB : f->logits;
-        TRY(gemv(&f->w.output, B, f->x, lg, S2P_FA_CB, GEMV_X_NORM, f->w.norm.data, f->ssq_a,
+        TRY(gemv(&f->w.output, B, x, lg, S2P_FA_CB, GEMV_X_NORM, f->w.norm.data, ssq,
                  GEMV_EPI_STORE, NULL, st));
         HIPCHK(s2pk_argmax((const s2p_bf16*)lg, f->stage + (size_t)(cb - 1) * B, B, S2P_FA_CB, st));
     }

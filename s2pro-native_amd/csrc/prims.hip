@@ -532,6 +532,39 @@ extern "C" hipError_t s2p_fa_embed_ssq_launch(const void* table, const int32_t* 
     return hipGetLastError();
 }
 
+/* The first pass of a frame, two rows a session: row 2 b = hidden[b], row
+ * 2 b + 1 = table[clamp(ids[b])], with their sums of squares. */
+__global__ __launch_bounds__(64) void k_fa_prime(const uint16_t* __restrict__ hidden,
+                                                 const uint16_t* __restrict__ table,
+                                                 const int32_t* __restrict__ ids, int n_ids,
+                                                 uint16_t* __restrict__ x, float* __restrict__ ssq,
+                                                 int width) {
+    const int m = blockIdx.y, blk = blockIdx.x, lane = threadIdx.x;
+    const uint16_t* src = hidden + (size_t)(m >> 1) * width;
+    if (m & 1) {
+        int id = ids[m >> 1];
+        id = id < 0 ? 0 : (id >= n_ids ? n_ids - 1 : id);
+        src = table + (size_t)id * width;
+    }
+    const int c = blk * 64 + lane;
+    const uint16_t v = src[c];
+    coh_st16(x + (size_t)m * width + c, v);
+    const float f = bf2f(v);
+    const float t = sum_lanes16(f * f);
+    if ((lane & 15) == 0) coh_stf(ssq + (size_t)(blk * 4 + (lane >> 4)) * 128 + m, t);
+}
+
+extern "C" hipError_t s2p_fa_prime_launch(const void* hidden, const void* table, const int32_t* ids,
+                                          int n_ids, void* x, float* ssq, int n_sess, int width,
+                                          hipStream_t st) {
+    if (n_sess <= 0) return hipSuccess;
+    if (width % 64) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_fa_prime, dim3(width / 64, 2 * n_sess), dim3(64), 0, st,
+                       (const uint16_t*)hidden, (const uint16_t*)table, ids, n_ids, (uint16_t*)x,
+                       ssq, width);
+    return hipGetLastError();
+}
+
 /* The 10-codebook VQ embedding of frame t added onto rows[t] (reference
  * fastar.h:46-52): codes [10][T] codebook-major, clamped to 0..4095; the ten
  * rows of table [10 * 4096][dim] summed in f32 in codebook order, rounded to

@@ -64,6 +64,9 @@ hipError_t s2p_qkrope_append_launch(const void* qkv, void* q_out, const void* qn
  * ([width/16][128]); the 10-codebook VQ embedding added onto rows. */
 hipError_t s2p_fa_embed_ssq_launch(const void* table, const int32_t* ids, int n_ids, void* x,
                                    float* ssq, int rows, int width, hipStream_t st);
+/* The frame's first two rows a session: hidden[b] and table[clamp(ids[b])] */
+hipError_t s2p_fa_prime_launch(const void* hidden, const void* table, const int32_t* ids, int n_ids,
+                               void* x, float* ssq, int n_sess, int width, hipStream_t st);
 /* Fast-AR attention (csrc/fa_attn.hip): RoPE, K/V append and attention of the
  * rows s * nn .. + nn - 1 of every session s at positions p0 .. p0 + nn - 1
  * (nn 1 or 2); rope: the (cos, sin) row of position p at p * rope_stride; kv:

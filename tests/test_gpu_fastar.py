@@ -293,6 +293,10 @@ def test_frame_rows_past_eight(lib, decoder):
             return bf16_vals(to_host(lg, np.uint16))[0].astype(np.float64)
 
         whole = frame(hid, sem, 12)
+        # eight sessions: the prime and first code rows in one pass of 16
+        eight = frame(hid[:8].contiguous(), sem[:8].contiguous(), 8)
+        d = np.linalg.norm(whole[:8] - eight, axis=1) / np.linalg.norm(eight, axis=1)
+        assert (d <= 2e-2).all(), d
         for i in range(0, 12, 4):
             part = frame(hid[i:i + 4].contiguous(), sem[i:i + 4].contiguous(), 4)
             d = np.linalg.norm(whole[i:i + 4] - part, axis=1) / np.linalg.norm(part, axis=1)
