@@ -182,6 +182,17 @@ __global__ __launch_bounds__(128) void k_attn_combine_bal(const float* __restric
 #define TR_VOFF(t, d) ((t) * 128 + ((((d) >> 3) ^ TR_VSW(t)) << 3) + ((d) & 7))
 #define TR_LDS_BYTES (4 * AT_TILE * 128 * 2)
 
+/* hi + lo bf16 pairs of two floats (16 significant bits), packed conversions:
+ * with a conversion per value the kernel spilled and took 51.7 us (4 sessions
+ * x 17 rows at 8,192 tokens), so 49 */
+S2P_DEV void pk_hilo(float a, float b, uint32_t& h, uint32_t& l) {
+    typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f2;
+    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 b2;
+    h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){a, b}, b2));
+    const f2 r = {a - __uint_as_float(h << 16), b - __uint_as_float(h & 0xFFFF0000u)};
+    l = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, b2));
+}
+
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_attn_tree(AttnArgs a) {
 #pragma clang fp contract(off)
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -291,21 +302,24 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         const float ms = mn == -INFINITY ? 0.f : mn;
         const float corr = __expf(m - ms);
         float ls = 0.f;
-        float p[2][4], lo[2][4];
+        float p[2][4];
 #pragma unroll
         for (int ps = 0; ps < 2; ps++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 p[ps][v] = __expf(t[ps][v] - ms);
                 ls += p[ps][v];
-                lo[ps][v] = p[ps][v] - bf2f(f2bf(p[ps][v]));
             }
         l = l * corr + ls;
         m = mn;
-        const s2p_u32x4 ph = {pk_bf(p[0][0], p[0][1]), pk_bf(p[0][2], p[0][3]),
-                              pk_bf(p[1][0], p[1][1]), pk_bf(p[1][2], p[1][3])};
-        const s2p_u32x4 pl = {pk_bf(lo[0][0], lo[0][1]), pk_bf(lo[0][2], lo[0][3]),
-                              pk_bf(lo[1][0], lo[1][1]), pk_bf(lo[1][2], lo[1][3])};
+        s2p_u32x4 ph, pl;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint32_t hw, lw;
+            pk_hilo(p[i >> 1][2 * (i & 1)], p[i >> 1][2 * (i & 1) + 1], hw, lw);
+            ph[i] = hw;
+            pl[i] = lw;
+        }
         if (__any(corr != 1.0f)) {
 #pragma unroll
             for (int dt = 0; dt < 8; dt++)

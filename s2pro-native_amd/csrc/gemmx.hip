@@ -381,21 +381,35 @@ __global__ __launch_bounds__(512) void k_gmx_pack(const uint16_t* __restrict__ x
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int ct = blockIdx.x;
     if constexpr (NORM) {
+        /* the wave's two rows, every load of up to 2560 k values in flight */
+        constexpr int NB = 5;
+        const uint16_t* xr[2];
+        float s[2] = {0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 2; j++) xr[j] = x + (size_t)min(16 * ct + 2 * wave + j, M - 1) * ldx;
+        for (int k0 = 0; k0 < K; k0 += 512 * NB) {
+            s2p_u32x4 v[2][NB];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+                    v[j][b] = *(const s2p_u32x4*)(xr[j] + min(k0 + 512 * b + 8 * lane, K - 8));
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    if (k0 + 512 * b + 8 * lane >= K) continue;
+#pragma unroll
+                    for (int d = 0; d < 4; d++) {
+                        s[j] = fmaf(bf2f_lo(v[j][b][d]), bf2f_lo(v[j][b][d]), s[j]);
+                        s[j] = fmaf(bf2f_hi(v[j][b][d]), bf2f_hi(v[j][b][d]), s[j]);
+                    }
+                }
+        }
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const int row = 2 * wave + j;
-            const uint16_t* xr = x + (size_t)min(16 * ct + row, M - 1) * ldx;
-            float s = 0.f;
-            for (int k = lane * 8; k < K; k += 512) {
-                const s2p_u32x4 v = *(const s2p_u32x4*)(xr + k);
-#pragma unroll
-                for (int d = 0; d < 4; d++) {
-                    s = fmaf(bf2f_lo(v[d]), bf2f_lo(v[d]), s);
-                    s = fmaf(bf2f_hi(v[d]), bf2f_hi(v[d]), s);
-                }
-            }
-            s = wave_sum_down(s);
-            if (lane == 0) s_inv[row] = rsqrt_rule(s / (float)K + eps);
+            const float t = wave_sum_down(s[j]);
+            if (lane == 0) s_inv[2 * wave + j] = rsqrt_rule(t / (float)K + eps);
         }
         __syncthreads();
     }
@@ -447,10 +461,11 @@ static hipError_t gx_launch(const GmxArgs& a, const GemvArgs& g, int t, int mtw,
                             hipStream_t st) {
     uint16_t* xp = (uint16_t*)a.x;
     const int nck = a.K / GX_CK;
-    /* about a workgroup a chunk and 16 rows: the pass is a round trip, not
-     * bandwidth; a norm reads its rows once a part */
+    /* a workgroup a chunk and 16 rows: the pass is a round trip, not bandwidth.
+     * A norm reads its rows once a workgroup: two chunks, a piece a thread
+     * (M = 40, K = 2560: 4.5 us; in eight parts with row sums load by load 6.7) */
     const bool norm = g.xmode == GEMV_X_NORM;
-    const dim3 pg((unsigned)a.mt, (unsigned)(norm ? (nck < 8 ? nck : 8) : (nck < 32 ? nck : 32)));
+    const dim3 pg((unsigned)a.mt, (unsigned)(norm ? (nck + 1) / 2 : (nck < 32 ? nck : 32)));
     if (norm)
         hipLaunchKernelGGL((k_gmx_pack<WFMT, true>), pg, dim3(512), 0, st, g.x, g.ldx, g.norm_w, xp,
                            a.M, a.K, a.mt, g.norm_eps);
