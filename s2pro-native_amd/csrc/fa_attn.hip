@@ -1,5 +1,5 @@
 /* s2pro MI355X — fast-AR attention: RoPE, K/V append and attention over the at
- * most S2P_FA_SEQ slots of a frame (reference fastar.c's attention step).
+ * most S2P_FA_SEQ slots of a frame (reference src/fastar/fastar.cu:647-789).
  *
  * What bounds it: one round trip to memory and the launch; a session's cache
  * is 11 slots.  So there are no tiles, no MFMA and no LDS: a wave is one query
