@@ -54,9 +54,9 @@
 #include "gemv_dev.h"
 #include "s2pro/gemm.h"
 
-/* whole-K workgroups of up to 16 waves, one column tile (M <= 16) */
-template <int WFMT>
-__global__ __launch_bounds__(1024) void k_gemv3(GemvArgs a) {
+/* whole-K workgroups of up to 16 waves (MT = 1: M <= 16) or 8 waves (MT = 2) */
+template <int WFMT, int MT>
+__global__ __launch_bounds__(MT == 1 ? 1024 : 512) void k_gemv3(GemvArgs a) {
     extern __shared__ __align__(16) unsigned char smem3[];
     /* every argument in one round of scalar loads: left to itself the
      * compiler issues them next to their first uses, three dependent
@@ -66,8 +66,8 @@ __global__ __launch_bounds__(1024) void k_gemv3(GemvArgs a) {
                  "s"(a.K), "s"(a.gps), "s"(a.ks), "s"(a.rt), "s"(a.xmode), "s"(a.epi),
                  "s"(a.ssq_in_blocks), "s"(a.norm_eps), "s"(gridDim.x));
     GvBuf b0, b1;
-    gv3_block<WFMT, 1, false, false, false, false>(a, blockIdx.x, gridDim.x,
-                                                  (LDS(unsigned char)*)smem3, a.y, b0, b1);
+    gv3_block<WFMT, MT, false, false, false, false>(a, blockIdx.x, gridDim.x,
+                                                   (LDS(unsigned char)*)smem3, a.y, b0, b1);
 }
 
 template <int WFMT, int MT, bool WIN1>
@@ -241,11 +241,13 @@ extern "C" hipError_t s2p_gemv_plan(GemvArgs* ap, int slots, dim3* grid_out, siz
  * hipErrorNotSupported when the activations do not fit in LDS (the split-K
  * engine runs instead). */
 extern "C" hipError_t s2p_gemv3_plan(GemvArgs* a, dim3* grid, dim3* block, size_t* lds_out) {
-    if (a->M > 16) return hipErrorNotSupported;
+    /* two column tiles: INT8 and bf16 (INT4 has k_gemm4 there) */
+    if (a->M > 32 || (a->M > 16 && a->wfmt == GEMV_W_INT4)) return hipErrorNotSupported;
     const int G = a->K >> 5;
+    const int mt = (a->M + 15) / 16;
     const bool swiglu = a->epi == GEMV_EPI_SWIGLU;
     const int tiles = swiglu ? (a->N >> 1) / 16 : (a->N + 15) / 16;
-    const int nwmax = 16;
+    const int nwmax = mt == 1 ? 16 : 8;
     const int chg = gv_chg(a->wfmt);
     const int cus = s2p_cu_count();
     const int kmax = swiglu ? nwmax / 2 : nwmax;
@@ -268,7 +270,7 @@ extern "C" hipError_t s2p_gemv3_plan(GemvArgs* a, dim3* grid, dim3* block, size_
         const int rt = per * units, nw = rt * ks;
         const int ngroups = (tiles + units - 1) / units;
         /* resident workgroups per CU: LDS, and waves at this kernel's
-         * register budget (16 waves per CU) */
+         * register budget (16 waves per CU at MT = 1, else 8) */
         const size_t lds1 = gv3_lds_bytes(a->M, gps, a->wfmt, ks, nw, 1);
         int per_cu = (int)(GV3_LDS_MAX / lds1);
         const int wcap = nwmax / nw;
@@ -292,16 +294,24 @@ extern "C" hipError_t s2p_gemv3_plan(GemvArgs* a, dim3* grid, dim3* block, size_
     }
 }
 
-template <int WFMT>
-static hipError_t gv3_launch(const GemvArgs& a, dim3 grid, dim3 block, size_t lds,
-                             hipStream_t st) {
+template <int WFMT, int MT>
+static hipError_t gv3_launch_mt(const GemvArgs& a, dim3 grid, dim3 block, size_t lds,
+                                hipStream_t st) {
     /* once per instantiation (thread-safe static initialisation) */
-    static const hipError_t attr = hipFuncSetAttribute((const void*)k_gemv3<WFMT>,
+    static const hipError_t attr = hipFuncSetAttribute((const void*)k_gemv3<WFMT, MT>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        GV3_LDS_MAX);
     (void)attr;
-    hipLaunchKernelGGL((k_gemv3<WFMT>), grid, block, lds, st, a);
+    hipLaunchKernelGGL((k_gemv3<WFMT, MT>), grid, block, lds, st, a);
     return hipGetLastError();
+}
+
+template <int WFMT>
+static hipError_t gv3_launch(const GemvArgs& a, dim3 grid, dim3 block, size_t lds,
+                             hipStream_t st) {
+    if constexpr (WFMT != GEMV_W_INT4)
+        if (a.M > 16) return gv3_launch_mt<WFMT, 2>(a, grid, block, lds, st);
+    return gv3_launch_mt<WFMT, 1>(a, grid, block, lds, st);
 }
 
 static hipError_t gemv_engines(const GemvArgs* ap, hipStream_t st) {

@@ -513,11 +513,14 @@ static s2p_status gemv_ex(const s2p_backbone* b, const s2p_linear* lin, int M, c
                           S2pQkvParts* parts, hipStream_t st) {
     GemvArgs a;
     gemv_args(&a, lin, M, x, ldx, y, ldy, xmode, norm_w, ssq_in, epi, ssq_out);
-    /* An appended INT8 / INT4 code is a rounded sum: another summation order
-     * moves about 5% of the codes from the second layer on (measured, 16
-     * rows, two layers).  Plans over quantised caches keep the engines, and
-     * the order, that the codes already in such caches were written with */
-    if (b->kvb != 16 && lin->q_packed) a.engine = GEMV_ENGINE_STAGED;
+    /* An appended INT8 / INT4 code is a whole number, a rounded sum: another
+     * summation order moves about 5% of the codes from the second layer on by
+     * one step (measured, 16 rows, two layers).  Plans over quantised caches
+     * stay on the staged engines, so that a plan of given rows and weights
+     * appends the same bytes, and returns the same logits, as it always has.
+     * (Only that: the order is not the same at every number of rows, k_mk2,
+     * k_gemv3, k_gemm4 and the split-K engine each have their own) */
+    if (b->kvb != 16) a.engine = GEMV_ENGINE_STAGED;
     int deferred = 0;
     if (M > 16 && M <= 96) {
         a.inv_in = inv_in;

@@ -94,6 +94,47 @@ def bf16_vals(bits):
     return (np.ascontiguousarray(bits, np.uint16).astype(np.uint32) << 16).view(np.float32)
 
 
+class GemvArgs(ctypes.Structure):
+    """The launch descriptor of csrc/gemv_internal.h (zero: plain, STORE, AUTO)."""
+    _fields_ = [("w", ctypes.c_void_p), ("s", ctypes.c_void_p), ("x", ctypes.c_void_p),
+                ("ldx", ctypes.c_int), ("y", ctypes.c_void_p), ("ldy", ctypes.c_int),
+                ("M", ctypes.c_int), ("N", ctypes.c_int), ("K", ctypes.c_int),
+                ("wfmt", ctypes.c_int), ("gps", ctypes.c_int), ("splits", ctypes.c_int),
+                ("win", ctypes.c_int), ("nrb", ctypes.c_int), ("ks", ctypes.c_int),
+                ("rt", ctypes.c_int), ("xmode", ctypes.c_int), ("norm_w", ctypes.c_void_p),
+                ("norm_eps", ctypes.c_float), ("ssq_in", ctypes.c_void_p),
+                ("ssq_in_blocks", ctypes.c_int), ("epi", ctypes.c_int),
+                ("ssq_out", ctypes.c_void_p), ("part", ctypes.c_void_p),
+                ("part_cap", ctypes.c_int64), ("counters", ctypes.c_void_p),
+                ("engine", ctypes.c_int), ("inv_in", ctypes.c_void_p),
+                ("inv_out", ctypes.c_void_p), ("inv_eps", ctypes.c_float),
+                ("deferred", ctypes.c_void_p)]
+
+
+GEMV_AUTO, GEMV_STAGED = 0, 1
+GEMV_STORE, GEMV_RESID, GEMV_SWIGLU = 0, 1, 2
+GEMV_FMT = {"int4": 0, "int8": 1, "bf16": 2}
+SSQ_ROWS = 128  # rows a block of sums of squares has room for
+
+
+def gemv_launch(lib, fmt, w, s, x, y, M, N, K, ldy=None, engine=GEMV_AUTO, epi=GEMV_STORE,
+                norm_w=None, ssq_in=None, ssq_out=None, eps=1e-6):
+    """s2p_gemv_launch on the library's scratch; w, s, x, y, ..: device
+    addresses; norm_w: with an input RMSNorm over rows of K"""
+    for f, r in (("part", ctypes.c_void_p), ("part_cap", ctypes.c_int64),
+                 ("counters", ctypes.c_void_p)):
+        getattr(lib, "s2p_gemm_ctx_" + f).restype = r
+    a = GemvArgs(w=w, s=s, x=x, ldx=K, y=y, ldy=N if ldy is None else ldy, M=M, N=N, K=K,
+                 wfmt=GEMV_FMT[fmt], epi=epi, engine=engine, ssq_out=ssq_out,
+                 part=lib.s2p_gemm_ctx_part(), part_cap=lib.s2p_gemm_ctx_part_cap(),
+                 counters=lib.s2p_gemm_ctx_counters())
+    if norm_w is not None:
+        a.xmode, a.norm_w, a.norm_eps, a.ssq_in, a.ssq_in_blocks = 1, norm_w, eps, ssq_in, K // 16
+    fn = lib.s2p_gemv_launch
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p]
+    s2pamd.hip_check(fn(ctypes.byref(a), S()), "gemv launch")
+
+
 def assert_close_rel(got, want, rel=1e-2, floor_frac=1e-2, what=""):
     """|got - want| <= rel * |want| + floor_frac * rms(want), elementwise."""
     got = np.asarray(got, np.float64)

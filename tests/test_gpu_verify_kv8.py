@@ -17,11 +17,12 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 import pyoracle as po
 import s2pamd
-from gpu_util import (P, S, assert_close_norm, bf16_bits, bf16_vals, d2h,
-                      empty, to_dev, to_host)
+from gpu_util import (GEMV_STAGED, P, S, SSQ_ROWS, assert_close_norm, bf16_bits, bf16_vals, d2h,
+                      empty, gemv_launch, to_dev, to_host)
 from test_gpu_verify import TREE16, host_layer, host_linear, make_backbone, plan
 from test_oracle_kv8 import decode
 
@@ -224,3 +225,40 @@ def test_kv_bits_rejected(lib):
     o = s2pamd.BackboneOpts(1, s2pamd.WQ_INT4, s2pamd.WQ_INT4, s2pamd.S2P_HEAD_SLICE, 8, 1, 64, 6)
     bb = ctypes.c_void_p()
     assert lib.s2p_backbone_create_random(ctypes.byref(o), 1, S(), ctypes.byref(bb)) != 0
+
+
+@pytest.mark.parametrize("quant", [s2pamd.WQ_INT8, s2pamd.WQ_INT4], ids=["int8w", "int4w"])
+@pytest.mark.parametrize("n,R", [(2, 5), (3, 8), (4, 8), (5, 8)])  # 10, 24, 32 and 40 rows
+def test_kv8_plans_keep_the_staged_engines(lib, quant, n, R):
+    """A plan over quantised caches runs its linears in the staged engines'
+    summation order whatever the weights' format: the q / k / v rows that its
+    codes are rounded from are those engines' bits."""
+    ctx, L, bw = 128, 40, 8
+    bb = make_backbone(lib, 1, quant, s2pamd.S2P_HEAD_SLICE, n * R, n, ctx, 5, kv_bits=bw)
+    try:
+        c = [new_kv8(lib, bb, 1, ctx, L, bw, 60 + i) for i in range(n)]
+        plan(lib, bb, [-1] + list(range(R - 1)), [d for d, _, _ in c], [L] * n,
+             scales=[s for _, _, s in c])
+        x = to_dev(bf16_bits(np.random.default_rng(n).standard_normal((n * R, 2560))
+                             .astype(np.float32)))
+        lg = empty((n * R, s2pamd.S2P_HEAD_SLICE))
+        s2pamd.check(lib.s2p_verify_forward(bb, P(x), P(lg), S()))
+        ptrs = [ctypes.c_void_p() for _ in range(5)]
+        dbg = lib.s2p_backbone_debug_ptrs
+        dbg.restype, dbg.argtypes = None, [ctypes.c_void_p] * 6
+        dbg(bb, *[ctypes.byref(p) for p in ptrs])
+        qkv = d2h(ptrs[1].value, n * R * 6144 * 2, np.uint16).reshape(n * R, 6144)
+        res, ssq = empty((n * R, 2560)), empty((160, SSQ_ROWS), torch.float32)
+        init = lib.s2p_resid_init_launch
+        init.restype = ctypes.c_int
+        init.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_int] * 2 + [ctypes.c_void_p]
+        s2pamd.hip_check(init(P(x), P(res), P(ssq), n * R, 2560, S()), "resid init")
+        layer = lib.s2p_backbone_layer(bb, 0).contents
+        lin, y = layer.wqkv, empty((n * R, 6144))
+        w, f = (lin.w_pack, "int4") if lin.q_packed else (lin.w_int8, "int8")
+        gemv_launch(lib, f, w.data, lin.w_iscale.data, P(res), P(y), n * R, 6144, 2560,
+                    engine=GEMV_STAGED, norm_w=layer.attn_norm.data, ssq_in=P(ssq))
+        want = to_host(y, np.uint16)
+        assert np.array_equal(qkv, want), f"{(qkv != want).sum()} q/k/v values differ"
+    finally:
+        lib.s2p_backbone_free(bb)
