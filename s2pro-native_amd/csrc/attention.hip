@@ -544,7 +544,7 @@ extern "C" hipError_t s2pk_attention_decode(const s2p_bf16* q, const s2p_bf16* c
                                             const int32_t* pos, int max_seq, int max_len,
                                             float* part, hipStream_t st) {
     if (rows <= 0) return hipSuccess;
-    if (head_dim != AT_HD || q_heads != 4 * kv_heads || !part || max_len <= 0)
+    if (head_dim != AT_HD || kv_heads <= 0 || q_heads != 4 * kv_heads || !part || max_len <= 0)
         return hipErrorInvalidValue;
     return s2p_attn_dec_launch((const uint16_t*)q, (const void* const*)k_caches,
                                (const void* const*)v_caches, nullptr, nullptr, (uint16_t*)out,

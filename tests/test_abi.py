@@ -62,6 +62,12 @@ def test_argument_validation(lib):
     # verify entry points on a null backbone
     assert lib.s2p_verify_forward(None, None, None, None) == S2P_ERR_INVALID
     assert lib.s2p_verify_step(None, None, 0, None) == S2P_ERR_INVALID
+    # attention without heads, or with a grouping the kernels do not have
+    p = 1 << 20  # never read
+    for qh, kvh in ((0, 0), (-4, -1), (32, 4)):
+        assert lib.s2pk_attention_decode(p, p, p, p, 1, qh, kvh, 128, p, 16, 16, p, None) != 0
+        assert lib.s2pk_attention8_decode(p, p, p, p, p, p, 1, qh, kvh, 128, p, 16, 16, None, 8,
+                                          None) != 0
     # the accept workspace size is a pure function
     assert lib.s2p_verify_accept_work_bytes(1, 5) > 0
     assert lib.s2p_verify_accept_work_bytes(8, 5) >= lib.s2p_verify_accept_work_bytes(1, 5)
