@@ -67,7 +67,10 @@ const s2pfa_weights* s2pfa_weights_of(const s2pfa* f);
 
 /* reference fastar.h:66-75.  hidden [B, 2560] device bf16 (final-normed),
  * sem_ids [B] HOST (0..4095); writes out_codes[b * 10 + 1 .. 9] (HOST),
- * leaves out_codes[b * 10] untouched; synchronises the stream. */
+ * leaves out_codes[b * 10] untouched; synchronises the stream.
+ * For B <= 8 a row's codes and logits are the same bits whatever rows run
+ * beside it and however many; above 8 the linears sum in another order (one
+ * up to 16 rows, others beyond), and two near-equal logits may change places. */
 s2p_status s2pfa_decode_frame_batch(s2pfa* f, const void* hidden, const int32_t* sem_ids, int B,
                                     int32_t* out_codes, hipStream_t st);
 /* reference fastar.h:77-83.  sem_dev [B] device; no sync: *stage_dev points

@@ -10,7 +10,7 @@
  * SwiGLU in its epilogue; w2 with the residual add.  The step input and the
  * prime pass's hidden enter through a gather / copy that also writes the
  * sums of squares.  Launches per frame of
- * up to 8 rows: 9 x (1 + 4 x 5 + head + argmax) + 1 (the prime rows go with the
+ * up to 4 rows: 9 x (1 + 4 x 5 + head + argmax) + 1 (the prime rows go with the
  * first code's); above that 1 + 4 x 5 more. */
 #include "s2pro/fastar.h"
 
@@ -38,7 +38,12 @@ unsigned* s2p_gemm_ctx_counters(void);
 #define FA_EPS 1e-6f
 #define FA_ROPE_BASE 1000000.0f
 #define FA_NPOS 10 /* positions 0 (prime) .. 9 */
-#define FA_BOTH 16 /* most rows of a pass over positions 0 and 1 together */
+/* most rows of a pass over positions 0 and 1 together: the GEMV's 8-row tiles.
+ * Its 16-row tiles sum K in another order, so frames of 5 to 8 sessions whose
+ * first pass had 10 to 16 rows gave other bits than the same rows beside fewer
+ * sessions; the draft's codes and their verification, made in batches of
+ * different sizes, are compared for equality */
+#define FA_BOTH 8
 
 struct s2pfa {
     s2pfa_weights w;
@@ -269,7 +274,7 @@ static s2p_status frame(s2pfa* f, const void* hidden, const int32_t* sem_dev, in
      * never read (the reference computes and discards them).  The row of
      * position 1, the semantic code's embedding, is known as well, so one pass
      * over the weights takes both rows of every session, hidden then code,
-     * while they are at most the 16 rows of a GEMV. */
+     * while they are at most FA_BOTH. */
     const int both = 2 * B <= FA_BOTH;
     if (!both) {
         HIPCHK(s2p_resid_init_launch(hidden, f->x, f->ssq_a, B, FA_DIM, st));
