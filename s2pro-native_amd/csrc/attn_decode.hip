@@ -19,12 +19,16 @@
  *     codes would have to be gathered byte by byte across slots, and the scale
  *     folded into P one group at a time;
  *     Planes need no alignment: global vector loads take any address;
+ *   - bf16 planes are loaded past the caches (nontemporal): each byte is read
+ *     once a call.  16 sessions at 8,192 tokens (537 MB) take 84 us, 97 with
+ *     cached loads; 64 at 2,048 83 against 96;
  *   - the lanes' sums fold once at the end (lane swaps that halve the values
  *     each step), the waves' states merge through LDS, the splits in
  *     k_attn_combine.
- * Measured (kernel + combine): 12 bf16 sessions of up to 4,096 tokens 32 us
- * (120 MB; the verify kernel with one row a segment 40), 8 INT8 sessions of up
- * to 8,192 tokens 32 us (the slot-a-thread kernel of kv8.hip 201). */
+ * Measured (kernel + combine), caches not resident: 12 bf16 sessions of 512 to
+ * 4,096 tokens 31 us (113 MB; the verify kernel with one row a segment 40), of
+ * 4,096 each 38 (44); 8 INT8 sessions of 1,024 to 8,192 tokens 35 us (the
+ * slot-a-thread kernel of kv8.hip 208). */
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -64,9 +68,10 @@ S2P_DEV AdPtr ad_base(const void* p, uint64_t off) {
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
     return (AdPtr)(((uint64_t)hi << 32) | lo);
 }
-template <class T>
+template <class T, bool NT = false>
 S2P_DEV T ad_at(AdPtr p, uint32_t off) {
-    return *(AD_GLOBAL(T)*)(p + off);
+    if constexpr (NT) return __builtin_nontemporal_load((AD_GLOBAL(T)*)(p + off));
+    else return *(AD_GLOBAL(T)*)(p + off);
 }
 
 /* 4 signed bytes -> 4 bf16 (exact) */
@@ -151,7 +156,7 @@ __global__ __launch_bounds__(64 * AD_WAVES) __attribute__((amdgpu_waves_per_eu(B
             const uint32_t slot = min((uint32_t)(tb + 16 * h + r), last);
 #pragma unroll
             for (int i = 0; i < Tile::NK; i++)
-                t.k[h][i] = ad_at<s2p_u32x4>(kb + 64 * i, slot * EL + 16u * q);
+                t.k[h][i] = ad_at<s2p_u32x4, BW == 16>(kb + 64 * i, slot * EL + 16u * q);
             if constexpr (BW != 16) { /* the lane's four slots of the scores */
 #pragma unroll
                 for (int i = 0; i < 4; i++)
@@ -167,7 +172,7 @@ __global__ __launch_bounds__(64 * AD_WAVES) __attribute__((amdgpu_waves_per_eu(B
                 t.v[i][0] = w.x;
                 t.v[i][1] = w.y;
             } else {
-                const s2p_u32x4 w = ad_at<s2p_u32x4>(vb, slot * EL + 16u * (lane % LPS));
+                const s2p_u32x4 w = ad_at<s2p_u32x4, BW == 16>(vb, slot * EL + 16u * (lane % LPS));
 #pragma unroll
                 for (int d = 0; d < 4; d++) t.v[i][d] = w[d];
             }
@@ -378,6 +383,39 @@ __global__ __launch_bounds__(64 * AD_WAVES) __attribute__((amdgpu_waves_per_eu(B
     }
 }
 
+/* Rounds a split of `units` rounds of (row, kv head) pairs, at most four
+ * blocks a CU (what fits at once).
+ * bf16: a tick's bytes are spread evenly when the CU with the most blocks has
+ * few rounds to do; a block costs about half a round besides, the combine a
+ * round and a twentieth a split, and one block a CU streams no faster than two
+ * do together.  The least such cost, of equals the fewest splits.  With four
+ * blocks a CU always, 64 sessions of 200 tokens took 15.5 us instead of 11.6
+ * and one of 32,768 took 50 instead of 36; with two, 24 sessions of 4,096 took
+ * 77 instead of 67.
+ * Quantised: about four blocks a CU, so that ragged lengths even out (32 INT4
+ * sessions of 512 to 4,096 tokens: 39 us, in two blocks a CU 49). */
+static int ad_rounds(int pairs, int units, bool bf16) {
+    const int cus = s2p_cu_count(), most = 4 * cus / pairs;
+    if (!bf16) {
+        const int ns = most < 1 ? 1 : most < units ? most : units;
+        return (units + ns - 1) / ns;
+    }
+    int best = units;
+    int64_t least = INT64_MAX;
+    for (int k = 1; k <= most || k == 1; k++) {
+        const int ups = (units + k - 1) / k, n = (units + ups - 1) / ups;
+        int64_t per_cu = ((int64_t)n * pairs + cus - 1) / cus;
+        if (per_cu < 2) per_cu = 2;
+        const int64_t cost = per_cu * (20 * (int64_t)ups + 10) + (n > 1 ? 20 + n : 0);
+        if (cost < least) {
+            least = cost;
+            best = ups;
+        }
+        if (ups == 1) break;
+    }
+    return best;
+}
+
 /* bw 16, 8 or 4; q_heads == 4 kv_heads.  part holds at least
  * ceil(max_len / 128) splits a (row, head); kss / vss: f16 scales (bw 8, 4) */
 extern "C" hipError_t s2p_attn_dec_launch(const uint16_t* q, const void* const* kcs,
@@ -398,13 +436,9 @@ extern "C" hipError_t s2p_attn_dec_launch(const uint16_t* q, const void* const* 
     a.qh = 4 * kv_heads;
     a.kvh_n = kv_heads;
     a.max_seq = max_seq;
-    /* splits of whole rounds of the block's tiles (128 slots): about four
-     * blocks a CU for the longest row's length, so that ragged lengths even out */
+    /* splits of whole rounds of the block's tiles (128 slots) */
     const int units = (max_len + AD_TILE * AD_WAVES - 1) / (AD_TILE * AD_WAVES);
-    int ns = 4 * s2p_cu_count() / (rows * kv_heads);
-    if (ns < 1) ns = 1;
-    if (ns > units) ns = units;
-    const int ups = (units + ns - 1) / ns;
+    const int ups = ad_rounds(rows * kv_heads, units, bw == 16);
     a.split_pos = ups * AD_TILE * AD_WAVES;
     a.nsplit = (units + ups - 1) / ups;
     const dim3 grid((unsigned)(rows * kv_heads), (unsigned)a.nsplit);
