@@ -4,7 +4,7 @@
  * and split-K flash-decode (kernels.cu:341-508), and adds the tree mask the
  * verify pass needs.  One kernel serves three callers:
  *   CONTIG  s2pk_attention: one contiguous cache, rows at positions pos..
- *           (8 waves a block, no scratch and so no position splits);
+ *           (4 or 8 waves a block, no scratch and so no position splits);
  *   PTRS    s2pk_attention_ptrs: per-row caches and positions (decode with the
  *           longest session known to the host is attn_decode.hip);
  *   PLAN    the verify forward: sessions x rows with per-row visibility
@@ -491,16 +491,24 @@ extern "C" hipError_t s2pk_attention(const s2p_bf16* q, const s2p_bf16* k_cache,
     a.max_seq = max_seq;
     /* No scratch, so no position splits: a workgroup's waves divide a segment's
      * positions.  Segments of four rows (one MFMA tile of query vectors) while
-     * they give at most a workgroup a CU, else of eight: a chunk of 128 rows at
-     * position 1787 takes 22 us in 256 workgroups of 8 waves, 32 in 128
-     * workgroups of 4 waves and eight rows. */
+     * they give at most a workgroup a CU, else of eight.  Eight waves where a
+     * CU has one workgroup and there are rounds of 32 positions for all of them:
+     * 128 rows at position 1787 take 24.8 us (four waves 25.7; eight rows and
+     * four waves 33.9), 128 at 100 8.6 (four waves 7.9), 4 at 0 6.3 (5.3); 256
+     * rows of eight at 4096 56 (four waves 66), at 100 13.2 (12.6).  With more
+     * workgroups than CUs four waves each are faster: 1024 rows at 0 take 43 us,
+     * in eight waves 62. */
     a.nsplit = 1;
     a.split_pos = max_seq; /* the whole cache: one split */
-    const bool four = (int64_t)((rows + 3) / 4) * kv_heads <= s2p_cu_count();
+    const int cus = s2p_cu_count(), span = pos + rows;
+    const bool four = (int64_t)((rows + 3) / 4) * kv_heads <= cus;
     a.nseg = four ? (rows + 3) / 4 : (rows + 7) / 8;
+    const bool one = (int64_t)a.nseg * kv_heads <= cus; /* a workgroup a CU */
     const dim3 grid((unsigned)(a.nseg * kv_heads));
-    if (four) attn_launch<1, 8, AM_CONTIG>(a, grid, st);
-    else attn_launch<2, 8, AM_CONTIG>(a, grid, st);
+    if (four && span >= 1536) attn_launch<1, 8, AM_CONTIG>(a, grid, st);
+    else if (four) attn_launch<1, AT_WAVES, AM_CONTIG>(a, grid, st);
+    else if (one && span >= 1024) attn_launch<2, 8, AM_CONTIG>(a, grid, st);
+    else attn_launch<2, AT_WAVES, AM_CONTIG>(a, grid, st);
     return hipGetLastError();
 }
 

@@ -246,10 +246,13 @@ def test_attention_decode_edges(lib, bw, lens):
             assert (np.abs(got[i, h] - want) <= bound).all(), (bw, L, h)
 
 
-# four- and eight-row segments (128 rows fill the 256 workgroups of four), a
-# wave's round (256 positions) and its edges
+# four- and eight-row segments (128 rows fill the 256 workgroups of four, 256
+# those of eight) of four and of eight waves, whose rounds are 128 and 256
+# positions, and the edges
 @pytest.mark.parametrize("rows,pos,max_seq", [(3, 0, 3), (4, 252, 256), (7, 250, 300),
-                                              (128, 129, 257), (129, 5, 160)])
+                                              (128, 129, 257), (129, 5, 160), (6, 1529, 1535),
+                                              (5, 1531, 1540), (130, 893, 1024), (131, 893, 1024),
+                                              (257, 800, 1057)])
 def test_attention_contig_segments(lib, rows, pos, max_seq):
     kc, vc = cache(rows + pos, max_seq)
     q = bf16_bits(np.random.default_rng(pos).standard_normal((rows, 4096)).astype(np.float32))
