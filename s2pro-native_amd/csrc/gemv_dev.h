@@ -722,7 +722,7 @@ __device__ void gv_fixup4(const GemvArgs& a, int rb, uint16_t* Y, int tid, int b
                  * 16 items a row, rows start at multiples of 16 lanes) */
                 ssq += __shfl_xor(ssq, 1, 64);
                 ssq += __shfl_xor(ssq, 2, 64);
-                if ((lane & 3) == 0 && ok) {
+                if ((lane & 3) == 0 && ok && n0 < nlim) { /* no block past the last output's */
                     float* sp = a.ssq_out + (size_t)(rb * 4 + (l4 >> 4)) * GEMV_MAX_M + m;
                     if (PLAIN) *sp = ssq;
                     else coh_stf(sp, ssq);

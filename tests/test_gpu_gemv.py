@@ -11,8 +11,8 @@ import torch
 
 import pyoracle as po
 import s2pamd
-from gpu_util import (P, S, assert_close_rel, bf16_bits, bf16_vals, empty, h2d_raw, to_dev,
-                      to_host)
+from gpu_util import (GEMV_RESID, GEMV_STORE, GEMV_SWIGLU, P, S, SSQ_ROWS, assert_close_rel,
+                      bf16_bits, bf16_vals, empty, gemv_launch, h2d_raw, sync, to_dev, to_host)
 
 pytestmark = pytest.mark.gpu
 
@@ -316,3 +316,94 @@ def test_g4_rms_inverse_rms(lib, M, blocks, K):
     got = to_host(inv, np.float32).astype(np.float64)
     exact = 1.0 / np.sqrt(ssq[:, :M].astype(np.float64).sum(axis=0) / K + eps)
     assert np.all(np.abs(got - exact) <= 2e-6 * exact), np.max(np.abs(got - exact) / exact)
+
+
+def fused_weights(fmt, N, K, seed):
+    """(codes, scales, binary64 weights, sum of |w| in the engine's terms) on the
+    device; INT4 products carry 24 x the scale besides w (the nibble's bias)"""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    if fmt == "int4":
+        w = torch.randint(0, 256, (N, K // 2), generator=g, device="cuda", dtype=torch.uint8)
+        s = (torch.rand(N, K // 32, generator=g, device="cuda") * 0.01).half()
+        b = w.to(torch.int16)
+        q = torch.stack([((b & 15) ^ 8) - 8, ((b >> 4) ^ 8) - 8], -1).reshape(N, K // 32, 32)
+        sd = s.double()[:, :, None]
+        return w, s, (q * sd).reshape(N, K), ((q.abs() + 24) * sd).reshape(N, K)
+    if fmt == "int8":
+        w = torch.randint(-128, 128, (N, K), generator=g, device="cuda", dtype=torch.int8)
+        s = torch.rand(N, generator=g, device="cuda") * 0.001
+        wf = w.double() * s.double()[:, None]
+        return w, s, wf, wf.abs() + 128 * s.double()[:, None]
+    w = (torch.randn(N, K, generator=g, device="cuda") / K ** 0.5).bfloat16()
+    return w, None, w.double(), w.double().abs()
+
+
+# every epilogue with and without the input norm, on each engine that the model's
+# calls reach: residuals of more tiles than workgroups (resident, streamed, K
+# split, several rounds), sums of squares of a last block that is not whole, SwiGLU
+# halves that do not divide
+SMALL = [("resid", 8212, 2560), ("resid", 8212, 4096), ("resid", 8212, 9728), ("resid", 2560, 9728),
+         ("norm", 4097, 2560), ("swiglu_norm", 8256, 2560), ("swiglu_norm", 19456, 2560)]
+LARGE = [("resid", 2564, 1152), ("resid", 12308, 512), ("norm", 6148, 640),
+         ("swiglu_norm", 8256, 640), ("swiglu_norm", 19456, 2560), ("swiglu", 8256, 1152)]
+
+
+@pytest.mark.parametrize("fmt", ["int4", "int8", "bf16"])
+@pytest.mark.parametrize("kind,N,K,Ms", [c + ((1, 8, 9, 16),) for c in SMALL] +
+                         [("swiglu", 8256, 4096, (1, 8))] +  # (9 bf16 rows: no engine)
+                         [c + ((17, 49, 97, 128),) for c in LARGE])
+def test_gemv_epilogues(lib, fmt, kind, N, K, Ms):
+    w, s, wf, wabs = fused_weights(fmt, N, K, N + K)
+    norm, epi = "norm" in kind, kind.split("_")[0]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    x = torch.randn(max(Ms), K, generator=g, device="cuda").bfloat16()
+    nw = (1 + 0.1 * torch.randn(K, generator=g, device="cuda")).bfloat16()
+    xe = x.float()
+    if norm:  # the rule's roundings; an inverse off by an ulp may turn a tie or two
+        inv = torch.rsqrt(x.double().square().mean(1, keepdim=True) + 1e-6).float()
+        xe = (xe * inv * nw.float()).bfloat16()
+    xe = xe.double()
+    acc = xe @ wf.T
+    # f32 sums (at most 64 additions deep per partial) and, with a norm, two
+    # elements one bf16 step off
+    err = 2.0 ** -18 * (xe.abs() @ wabs.T)
+    if norm:
+        err = err + 2.0 ** -7 * xe.abs().amax(1, keepdim=True) * wf.abs().amax(1)[None, :]
+    width = N // 2 if epi == "swiglu" else N
+    old = torch.randn(max(Ms), width, generator=g, device="cuda").bfloat16()
+    if epi == "swiglu":
+        gv, uv = acc[:, :width], acc[:, width:]
+        eg, eu = (2.0 ** -8 * v.abs() + e for v, e in ((gv, err[:, :width]), (uv, err[:, width:])))
+        sil = gv * torch.sigmoid(gv)
+        exact = sil * uv
+        # silu's slope is at most 1.1; its own rounding 2^-8
+        err = (1.1 * eg + 2.0 ** -8 * sil.abs()) * (uv.abs() + eu) + sil.abs() * eu
+    elif epi == "resid":
+        exact = old.double() + acc
+        err = err + 2.0 ** -8 * acc.abs()
+    else:
+        exact = acc
+    for M in Ms:
+        xm = x[:M].contiguous()
+        ssq_in = xm.float().square().view(M, K // 16, 16).sum(2).T  # [block][row]
+        si = torch.zeros(K // 16, SSQ_ROWS, device="cuda")
+        si[:, :M] = ssq_in
+        so = torch.full(((N + 15) // 16, SSQ_ROWS), -1.0, device="cuda")
+        y = old[:M].clone()
+        gemv_launch(lib, fmt, P(w), None if s is None else P(s), P(xm), P(y), M, N, K, ldy=width,
+                    epi={"resid": GEMV_RESID, "norm": GEMV_STORE, "swiglu": GEMV_SWIGLU}[epi],
+                    norm_w=P(nw) if norm else None, ssq_in=P(si) if norm else None,
+                    ssq_out=P(so) if epi == "resid" else None)
+        sync()
+        d = (y.double() - exact[:M]).abs()
+        bound = 2.0 ** -8 * exact[:M].abs() + err[:M]
+        bad = (d > bound).nonzero()
+        assert len(bad) == 0, (fmt, M, len(bad), bad[:4].tolist(), (d / bound).max().item())
+        if epi == "resid":
+            sq = torch.zeros(M, (N + 15) // 16 * 16, device="cuda", dtype=torch.float64)
+            sq[:, :N] = y.double().square()
+            want = sq.view(M, -1, 16).sum(2).T
+            assert torch.allclose(so[:, :M].double(), want, rtol=2.0 ** -20, atol=0), (fmt, M)
+            assert (so[:, M:] == -1.0).all()  # no row past M
