@@ -484,6 +484,32 @@ static hipError_t gx_launch(const GmxArgs& a, const GemvArgs& g, int t, int mtw,
     return hipGetLastError();
 }
 
+/* shapes in reach of this GEMM that another engine runs faster (M from 17 on,
+ * weights not resident, merges and packing included) */
+static bool gx_other(const GemvArgs& g) {
+    const int64_t km = (int64_t)g.K * g.M;
+    if (g.wfmt == GEMV_W_BF16) /* one launch of k_gemv3 against two and the merge: N = K = 1024,
+                                * M = 17 8.1 us against 10.2, M = 32 10.0 and 10.3; N = 6144,
+                                * M = 17 11.2 and 10.9; K = 512, N = 4096, M = 17 7.8 and 8.3 */
+        return g.N <= 4096 && g.K >= 512 && g.K <= 1024 && g.M <= (g.K > 512 ? 32 : 20);
+    if (g.wfmt != GEMV_W_INT4 || g.M > 96) return false;
+    /* INT4 at M <= 96: k_gemm4, which stages the row-major activations itself.
+     * Few rows, whose K both split: at M = 40 wqkv 16 us against 18, w2 20.4
+     * against 20.5 (with the merges; gate_up 33.5 against 27.8) */
+    if (g.N < GX_MIN_ROWS) return true;
+    /* little K: the packing launch shows (K = 512, N = 19456, M = 17: 7.0 against
+     * 9.0; M = 64: 12.7 and 11.9; K = 1024, N = 18742, M = 17: 10.1 against 11.1) */
+    if (km <= 512 * 24 || (g.N > 16384 && km <= 1024 * 33)) return true;
+    /* k_gemm4 still in one round where six tiles a CU are two here (K = 2560, N =
+     * 30000: M = 17 21.5 us against 27.0, M = 96 48.1 and 48.0), in two where they
+     * are three (N = 60000: M = 17 40.6 against 46.5, M = 80 87.4 and 91.0, M = 96
+     * 94.5 and 90.9), and with two activation tiles in five where they are seven
+     * (the head's 155776 rows: M = 17 97.9 against 102.7) */
+    const int cus = s2p_cu_count();
+    const int r = (g.N + 96 * cus - 1) / (96 * cus), r4 = (g.N + 128 * cus - 1) / (128 * cus);
+    return r > r4 && (r == 2 || (r == 3 && g.M <= 80) || (5 * r >= 7 * r4 && g.M <= 24));
+}
+
 /* 16 < M <= 128, K a multiple of 128; part holds the packed activations
  * (16 ceil(M / 16) x K bf16) and then the K splits' partials.
  * hipErrorNotSupported otherwise. */
@@ -492,11 +518,7 @@ extern "C" hipError_t s2p_gmx_launch(const GemvArgs* ap, hipStream_t st) {
     if (g.M <= 16 || g.M > GEMV_MAX_M || (g.K & 127) || g.N <= 0 || !g.part)
         return hipErrorNotSupported;
     const bool swiglu = g.epi == GEMV_EPI_SWIGLU;
-    /* INT4 at M <= 96 with few rows stays with k_gemm4, whose K splits stage
-     * the row-major activations themselves: at M = 40 wqkv 16 us against 18,
-     * w2 20.4 against 20.5 (with the merges; gate_up 33.5 against 27.8) */
-    if (g.wfmt == GEMV_W_INT4 && g.M <= 96 && g.N < GX_MIN_ROWS)
-        return hipErrorNotSupported;
+    if (gx_other(g)) return hipErrorNotSupported;
     GmxArgs a = {};
     a.w = g.w;
     a.s = g.s;
@@ -520,26 +542,35 @@ extern "C" hipError_t s2p_gmx_launch(const GemvArgs* ap, hipStream_t st) {
     a.rg = 2;
     int t;
     int rounds = 1;
+    /* activation tiles: up to four a wave (three beside three weight tiles),
+     * else in groups of waves; the waves left over are K slices */
+    auto wave_grid = [&]() {
+        const int mw = t == 3 ? 3 : 4;
+        a.mg = a.mt <= mw ? 1 : a.mt <= 2 * mw ? 2 : 4;
+        a.kw = GX_WAVES / (a.rg * a.mg);
+    };
     if (swiglu || tiles16 >= tmax * cus) {
         /* enough rows: one round of workgroups over the whole of K, dealt out
          * evenly, or as few rounds as the tiles allow */
         const int per_cu = (tiles16 + cus - 1) / cus, most = swiglu ? tmax : 2 * tmax;
         rounds = (per_cu + most - 1) / most;
         int ot = (per_cu + rounds - 1) / rounds;
-        if (!swiglu && ot == 1) a.rg = 1;
         t = swiglu ? ot : (ot + a.rg - 1) / a.rg;
         ot = swiglu ? t : t * a.rg;
         a.rpt = g.epi == GEMV_EPI_RESID /* tiles of the sums' 16 columns */
                     ? 16
                     : ((rows + cus * rounds - 1) / (cus * rounds) + ot - 1) / ot;
         a.splits = 1;
+        wave_grid();
     } else {
         /* few rows: blocks of 2 t tiles, K split over the remaining workgroups */
         t = tiles16 >= 256 ? tmax : 2;
         a.rpt = 16;
+        wave_grid();
         const int blocks = (tiles16 + 2 * t - 1) / (2 * t);
         int sp = cus / blocks;
-        if (sp > nck) sp = nck;
+        if (sp > nck / a.kw) sp = nck / a.kw; /* a chunk for each of a workgroup's K slices: INT8, 17
+                                           * rows, N = 512, K = 4096 in 8 splits 11.2 us, in 32 17.0 */
         if (sp < 1) sp = 1;
         a.np = (g.N + 3) & ~3;
         while (sp > 1 && xf + (int64_t)sp * g.M * a.np > g.part_cap) sp--;
@@ -548,12 +579,7 @@ extern "C" hipError_t s2p_gmx_launch(const GemvArgs* ap, hipStream_t st) {
     const int ot = swiglu ? t : t * a.rg;
     const int tiles = (rows + a.rpt - 1) / a.rpt;
     a.groups = (tiles + ot - 1) / ot;
-    /* activation tiles: up to four a wave (three beside three weight tiles),
-     * else in groups of waves */
-    const int mw = t == 3 ? 3 : 4;
-    a.mg = a.mt <= mw ? 1 : a.mt <= 2 * mw ? 2 : 4;
     const int mtw = (a.mt + a.mg - 1) / a.mg;
-    a.kw = GX_WAVES / (a.rg * a.mg);
     const dim3 grid((unsigned)(a.groups < cus ? a.groups : cus), (unsigned)a.splits);
     switch (g.wfmt) {
         case GEMV_W_INT4: return gx_launch<GEMV_W_INT4>(a, g, t, mtw, grid, st);

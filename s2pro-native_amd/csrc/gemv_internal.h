@@ -87,5 +87,7 @@ hipError_t s2p_gemv_generic_launch(int fmt, const void* w, const void* sc,
 }
 /* work decomposition for `slots` resident workgroups (gemv.hip) */
 extern "C" hipError_t s2p_gemv_plan(GemvArgs* a, int slots, dim3* grid, size_t* lds);
+/* the whole-K engine's; hipErrorNotSupported where the activations do not fit */
+extern "C" hipError_t s2p_gemv3_plan(GemvArgs* a, dim3* grid, dim3* block, size_t* lds);
 #endif
 #endif

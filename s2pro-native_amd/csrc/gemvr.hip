@@ -671,8 +671,31 @@ struct GvrClass<GEMV_W_BF16> {
     static constexpr int U1 = 4, NT1 = 6, NTW1 = 2, NTN1 = 1, U2 = 8, NT2 = 3, NTW2 = 1, U3 = 0;
 };
 
+/* streamed calls that another engine runs faster (weights not resident) */
+template <int WFMT>
+static bool gr_other(const GemvArgs& g, const GvrArgs& a, int cus) {
+    const int64_t kq = a.K >> 8;
+    const bool few = WFMT != GEMV_W_BF16 && a.groups <= 16 && kq >= 38 && kq * kq * a.M >= 16000;
+    const bool many = WFMT == GEMV_W_INT4 && a.K <= 8192 &&
+                      (a.groups + cus - 1) / cus * a.M >= 16;
+    if (!few && !many) return false;
+    GemvArgs t = g;
+    dim3 grid, block;
+    size_t lds;
+    const bool staged = s2p_gemv3_plan(&t, &grid, &block, &lds) == hipSuccess;
+    /* few workgroups, each with a long K to itself, where k_gemv3 does not hold
+     * the activations either: the split-K engine (INT8, N = 64: K = 12288, M = 8
+     * 12.6 us against 13.6, M = 16 15.1 and 18.7; K = 9728, M = 16 14.6 and 16.0) */
+    if (few && !staged) return true;
+    /* several rounds of 16 INT4 rows and many activation rows, whose loads come
+     * again with each round, while k_gemv3 keeps them in LDS, one chunk of K a
+     * wave (K = 5120: N = 20000, M = 9 26.8 us against 33.5, M = 4 24.7 and 26.7;
+     * N = 8192, M = 8 13.7 and 13.9, M = 4 12.6 and 11.8) */
+    return many && staged;
+}
+
 template <int WFMT, bool WIDE>
-static hipError_t gr_launch(GvrArgs& a, bool norm, hipStream_t st) {
+static hipError_t gr_launch(const GemvArgs& g, GvrArgs& a, bool norm, hipStream_t st) {
     typedef GvrClass<WFMT> Cl;
     const int units = a.K / gr_uk(WFMT), cus = s2p_cu_count();
     const bool swiglu = a.epi == GEMV_EPI_SWIGLU;
@@ -706,6 +729,7 @@ static hipError_t gr_launch(GvrArgs& a, bool norm, hipStream_t st) {
     const int tiles = (rows + a.rpt - 1) / a.rpt;
     a.groups = (tiles + ot - 1) / ot;
     const int grid = a.groups < cus ? a.groups : cus, nt = ot * per;
+    if (cls == 0 && gr_other<WFMT>(g, a, cus)) return hipErrorNotSupported;
     if constexpr (!WIDE && Cl::U3 > 0) /* 16 rows a workgroup, one round */
         if (cls == 0 && units > 16 * (Cl::U3 - 1) && units <= 16 * Cl::U3 && a.groups == grid)
             return gr_run<WFMT, 16, Cl::U3, 2, false, false, true>(a, grid, st);
@@ -719,8 +743,8 @@ static hipError_t gr_launch(GvrArgs& a, bool norm, hipStream_t st) {
 }
 
 template <int WFMT>
-static hipError_t gr_launch_m(GvrArgs& a, bool norm, hipStream_t st) {
-    return a.M <= 8 ? gr_launch<WFMT, false>(a, norm, st) : gr_launch<WFMT, true>(a, norm, st);
+static hipError_t gr_launch_m(const GemvArgs& g, GvrArgs& a, bool norm, hipStream_t st) {
+    return a.M <= 8 ? gr_launch<WFMT, false>(g, a, norm, st) : gr_launch<WFMT, true>(g, a, norm, st);
 }
 
 extern "C" hipError_t s2p_gvr_launch(const GemvArgs* ap, hipStream_t st) {
@@ -746,8 +770,8 @@ extern "C" hipError_t s2p_gvr_launch(const GemvArgs* ap, hipStream_t st) {
     a.norm_eps = g.norm_eps;
     const bool norm = g.xmode == GEMV_X_NORM;
     switch (g.wfmt) {
-        case GEMV_W_INT4: return gr_launch_m<GEMV_W_INT4>(a, norm, st);
-        case GEMV_W_INT8: return gr_launch_m<GEMV_W_INT8>(a, norm, st);
-        default: return gr_launch_m<GEMV_W_BF16>(a, norm, st);
+        case GEMV_W_INT4: return gr_launch_m<GEMV_W_INT4>(g, a, norm, st);
+        case GEMV_W_INT8: return gr_launch_m<GEMV_W_INT8>(g, a, norm, st);
+        default: return gr_launch_m<GEMV_W_BF16>(g, a, norm, st);
     }
 }

@@ -106,7 +106,9 @@ def test_int4p_gemm_six_tiles_repeat(lib, M, N, K):
 # do not divide, the streamed and the resident K classes, K with idle waves
 @pytest.mark.parametrize("fmt", ["int4", "int8", "bf16"])
 @pytest.mark.parametrize("N,K", [(5, 2560), (4097, 2560), (19461, 2560), (2567, 4096),
-                                 (2560, 9728), (4103, 9728), (33, 512), (9, 1024)])
+                                 (2560, 9728), (4103, 9728), (33, 512), (9, 1024),
+                                 # streamed calls that go to k_gemv3 and to the split-K engine
+                                 (8200, 4608), (64, 12288)])
 def test_gemv_small_m(lib, fmt, N, K):
     r = np.random.default_rng(N + K)
     if fmt == "int4":
@@ -150,7 +152,7 @@ def test_gemv_small_m(lib, fmt, N, K):
 # groups of one, two and four), rows that do not divide, K splits and none
 @pytest.mark.parametrize("fmt", ["int4", "int8", "bf16"])
 @pytest.mark.parametrize("N,K", [(12289, 512), (4097, 2560), (70, 1152), (2567, 9728), (5, 128),
-                                 (40003, 256)])
+                                 (40003, 256), (1031, 1024), (25003, 1280)])
 def test_linear_large_m(lib, fmt, N, K):
     r = np.random.default_rng(N * 3 + K)
     lin = s2pamd.Linear()
@@ -177,7 +179,7 @@ def test_linear_large_m(lib, fmt, N, K):
     xh = bf16_bits(r.standard_normal((128, K)).astype(np.float32))
     xd = to_dev(xh)
     exact = bf16_vals(xh).astype(np.float64) @ wf.T
-    for M in (17, 48, 49, 65, 96, 97, 113, 128):
+    for M in (17, 32, 48, 49, 65, 96, 97, 113, 128):
         y = empty((M, N))
         s2pamd.check(lib.s2p_linear_forward(ctypes.byref(lin), P(xd), P(y), M,
                                             0 if fmt == "bf16" else 2, S()), fmt)
