@@ -510,15 +510,19 @@ static bool gx_other(const GemvArgs& g) {
     return r > r4 && (r == 2 || (r == 3 && g.M <= 80) || (5 * r >= 7 * r4 && g.M <= 24));
 }
 
-/* 16 < M <= 128, K a multiple of 128; part holds the packed activations
- * (16 ceil(M / 16) x K bf16) and then the K splits' partials.
- * hipErrorNotSupported otherwise. */
+/* the calls that this GEMM takes: 16 < M <= 128, K a multiple of 128, room for
+ * the packed activations (16 ceil(M / 16) x K bf16) in part */
+extern "C" int s2p_gmx_takes(const GemvArgs* g) {
+    return g->M > 16 && g->M <= GEMV_MAX_M && !(g->K & 127) && g->N > 0 && g->part &&
+           (int64_t)((g->M + 15) / 16) * 8 * g->K <= g->part_cap && !gx_other(*g);
+}
+
+/* hipErrorNotSupported where it does not; part holds the packed activations and
+ * then the K splits' partials */
 extern "C" hipError_t s2p_gmx_launch(const GemvArgs* ap, hipStream_t st) {
     const GemvArgs& g = *ap;
-    if (g.M <= 16 || g.M > GEMV_MAX_M || (g.K & 127) || g.N <= 0 || !g.part)
-        return hipErrorNotSupported;
+    if (!s2p_gmx_takes(ap)) return hipErrorNotSupported;
     const bool swiglu = g.epi == GEMV_EPI_SWIGLU;
-    if (gx_other(g)) return hipErrorNotSupported;
     GmxArgs a = {};
     a.w = g.w;
     a.s = g.s;
@@ -532,7 +536,6 @@ extern "C" hipError_t s2p_gmx_launch(const GemvArgs* ap, hipStream_t st) {
     a.mt = (g.M + 15) / 16;
     a.x = (const uint16_t*)g.part;
     const int64_t xf = (int64_t)a.mt * 8 * g.K; /* floats of the packed activations */
-    if (xf > g.part_cap) return hipErrorNotSupported;
     a.part = g.part + xf;
     const int cus = s2p_cu_count(), nck = g.K / GX_CK;
     const int rows = swiglu ? g.N >> 1 : g.N;

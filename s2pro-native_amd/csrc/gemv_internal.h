@@ -65,6 +65,8 @@ typedef struct {
 hipError_t s2p_gemv_launch(const GemvArgs* a, hipStream_t st);
 /* 16 < M <= 128 (gemmx.hip); hipErrorNotSupported outside its shapes */
 hipError_t s2p_gmx_launch(const GemvArgs* a, hipStream_t st);
+/* whether it takes the call (engine GEMV_ENGINE_AUTO) */
+int s2p_gmx_takes(const GemvArgs* a);
 /* INT4, 16 < M <= 96 (gemm4.hip); hipErrorNotSupported outside that range */
 hipError_t s2p_gemm4_launch(const GemvArgs* a, hipStream_t st);
 /* M <= 16 (gemvr.hip); hipErrorNotSupported outside its shapes */

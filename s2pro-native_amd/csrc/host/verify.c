@@ -504,9 +504,18 @@ static void gemv_args(GemvArgs* ap, const s2p_linear* lin, int M, const void* x,
     *ap = a;
 }
 
+/* whether the normed GEMV of M rows over lin reads its rows' inverse RMS: k_gemm4
+ * does (INT4, 16 < M <= 96), the other engines take it from the rows themselves */
+static int reads_inv(const s2p_backbone* b, const s2p_linear* lin, int M) {
+    if (!lin->q_packed || M <= 16 || M > 96) return 0;
+    GemvArgs a;
+    gemv_args(&a, lin, M, NULL, lin->in_features, NULL, lin->out_features, GEMV_X_NORM, NULL, NULL,
+              GEMV_EPI_STORE, NULL);
+    return b->kvb != 16 || !s2p_gmx_takes(&a);
+}
+
 /* inv_out / inv_in: the output rows' inverse RMS written by a residual GEMV
- * for the normed GEMV that reads them next (the row-split INT4 GEMM at
- * 16 < M <= 96 only: elsewhere the consumer computes its own) */
+ * for the normed GEMV that reads them next (NULL: that one does not) */
 static s2p_status gemv_ex(const s2p_backbone* b, const s2p_linear* lin, int M, const void* x, int ldx, void* y,
                           int ldy, int xmode, const void* norm_w, const float* ssq_in, int epi,
                           float* ssq_out, const float* inv_in, float* inv_out,
@@ -659,19 +668,20 @@ s2p_status s2p_verify_forward(s2p_backbone* b, const void* x_in, void* logits, h
     float* ssq_b = b->ssq + (S2P_DIM / GEMV_SSQ_COLS) * GEMV_MAX_M;
     float* inv_a = b->ssq + 2 * (S2P_DIM / GEMV_SSQ_COLS) * GEMV_MAX_M;
     float* inv_b = inv_a + GEMV_MAX_M;
-    /* the inverse RMS goes from a residual GEMM to the next norm where both run
-     * on k_gemm4; the other engines take it from the rows themselves */
-    if (b->o.quant != S2P_WQ_INT4_G32 || M <= 16 || M > 96) inv_a = inv_b = NULL;
     S2P_TRY(hip_ok(s2p_resid_init_launch(x_in, b->x, ssq_a, M, S2P_DIM, st), "resid init"));
+    float* inv_in = NULL; /* of the rows of x, from the layer before */
     for (int l = 0; l < b->o.n_layers; l++) {
         const s2p_slow_layer* L = &b->layers[l];
+        const s2p_linear* next = l + 1 < b->o.n_layers ? &b->layers[l + 1].wqkv : &b->head;
+        float* inv_ffn = reads_inv(b, &L->gate_up, M) ? inv_b : NULL;
+        float* inv_next = reads_inv(b, next, M) ? inv_a : NULL;
         /* trees over bf16 caches: the qk-norm / RoPE / append kernel merges
          * wqkv's K-split partials itself (one launch fewer; the fused
          * attention prologue of the other plans measured slower reading them:
          * every split's blocks reread the partials) */
         S2pQkvParts qp = {NULL, 0, 0, 0};
         S2P_TRY(gemv_ex(b, &L->wqkv, M, b->x, S2P_DIM, b->qkv, S2P_QKV_WIDTH, GEMV_X_NORM,
-                        L->attn_norm.data, ssq_a, GEMV_EPI_STORE, NULL, l > 0 ? inv_a : NULL,
+                        L->attn_norm.data, ssq_a, GEMV_EPI_STORE, NULL, inv_in,
                         NULL, b->kvb == 16 && b->tree ? &qp : NULL, st));
         if (b->kvb != 16) {
             /* quantised caches: prologue + quantise-on-append, then the
@@ -701,15 +711,15 @@ s2p_status s2p_verify_forward(s2p_backbone* b, const void* x_in, void* logits, h
                                                   NORM_EPS, NULL, st),
                        "attention"));
         S2P_TRY(gemv(b, &L->wo, M, b->attn, S2P_Q_HEADS * S2P_HEAD_DIM, b->x, S2P_DIM, GEMV_X_PLAIN,
-                     NULL, NULL, GEMV_EPI_RESID, ssq_b, NULL, inv_b, st));
+                     NULL, NULL, GEMV_EPI_RESID, ssq_b, NULL, inv_ffn, st));
         S2P_TRY(gemv(b, &L->gate_up, M, b->x, S2P_DIM, b->gu, S2P_FFN_DIM, GEMV_X_NORM,
-                     L->ffn_norm.data, ssq_b, GEMV_EPI_SWIGLU, NULL, inv_b, NULL, st));
+                     L->ffn_norm.data, ssq_b, GEMV_EPI_SWIGLU, NULL, inv_ffn, NULL, st));
         S2P_TRY(gemv(b, &L->w2, M, b->gu, S2P_FFN_DIM, b->x, S2P_DIM, GEMV_X_PLAIN, NULL, NULL,
-                     GEMV_EPI_RESID, ssq_a, NULL, inv_a, st));
+                     GEMV_EPI_RESID, ssq_a, NULL, inv_next, st));
+        inv_in = inv_next;
     }
     return gemv(b, &b->head, M, b->x, S2P_DIM, logits, b->head.out_features, GEMV_X_NORM,
-                b->final_norm.data, ssq_a, GEMV_EPI_STORE, NULL, b->o.n_layers > 0 ? inv_a : NULL,
-                NULL, st);
+                b->final_norm.data, ssq_a, GEMV_EPI_STORE, NULL, inv_in, NULL, st);
 }
 
 /* ------------------------------------------------------------ acceptance */
