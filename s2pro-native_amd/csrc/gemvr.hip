@@ -654,13 +654,15 @@ static hipError_t gr_nt(const GvrArgs& a, int nt, int grid, hipStream_t st) {
 /* resident classes, the model's widths (every wave the same number U of whole
  * units, no checks between the tiles' multiplies): 1: K = 2560 on 10 waves;
  * 2: K = 4096 on 8.  A longer K streams.  NT / NTW / NTN: most tiles a round that
- * the registers hold, narrow / WIDE / WIDE with a norm.  U3: units a wave of
- * 16 waves that hold a longer K (w2's 9728) whole, two tiles, one round */
+ * the registers hold, narrow / WIDE / WIDE with a norm (a fourth INT4 WIDE tile
+ * spills: a layer of 10 rows 2.2 us longer, the full head at 9 rows 50.1 us
+ * instead of 48.5).  U3: units a wave of 16 waves that hold a longer K (w2's
+ * 9728) whole, two tiles, one round */
 template <int WFMT>
 struct GvrClass;
 template <>
 struct GvrClass<GEMV_W_INT4> {
-    static constexpr int U1 = 1, NT1 = 10, NTW1 = 4, NTN1 = 4, U2 = 2, NT2 = 6, NTW2 = 2, U3 = 3;
+    static constexpr int U1 = 1, NT1 = 10, NTW1 = 3, NTN1 = 3, U2 = 2, NT2 = 6, NTW2 = 2, U3 = 3;
 };
 template <>
 struct GvrClass<GEMV_W_INT8> {
