@@ -338,9 +338,9 @@ def main():
             abytes = sum(2 * M * (lin.in_features + lin.out_features) for lin in lins)
             per_launch = (wbytes + abytes) / len(lins)
             kern_gbs = per_launch / avg_launch_s / 1e9
-            # M <= 16 rows run on the GEMV engine, 16 < M <= 96 on k_gemm4
-            mt = (M + 15) // 16
-            kern_name = ((f"k_gemv3<INT4, MT={mt}>" if M <= 16 else f"k_gemm4<MT={mt}>") +
+            # M <= 16 rows run on the resident / streamed GEMV, 16 < M <= 96 on k_gemm4
+            # (gate_up and the head on k_gmx)
+            kern_name = (("k_gvr, k_gvs" if M <= 16 else "k_gemm4, k_gmx") +
                          " (all 145 weight GEMVs of a step, layer path)")
         lib.s2p_backbone_free(bb)
 

@@ -69,7 +69,7 @@ extern "C" hipError_t s2p_at_probe_get(uint64_t* host, int n) {
  * batch cut to its longest session's split count leaves most blocks of the
  * short sessions empty and the others long: eight sessions of 256 .. 4096
  * tokens ran 192 working blocks of up to 8 rounds (43 us); in splits of 3
- * rounds over up to 512 blocks they take 23, most of it the K/V stream and
+ * rounds over up to 512 blocks they take 31, most of it the K/V stream and
  * the 6 us prologue.  Returns u; cnt: the splits of the lane's segment, end:
  * of it and those before. */
 static __device__ __forceinline__ int wave_sum_i(int v) {
@@ -533,13 +533,6 @@ extern "C" hipError_t s2pk_attention_ptrs(const s2p_bf16* q, const s2p_bf16* con
     a.max_seq = max_seq;
     return attn_run(a, rows, 1, max_seq, 0, st);
 }
-
-/* attn_decode.hip */
-extern "C" hipError_t s2p_attn_dec_launch(const uint16_t* q, const void* const* kcs,
-                                          const void* const* vcs, const uint16_t* const* kss,
-                                          const uint16_t* const* vss, uint16_t* out, int rows,
-                                          int kv_heads, const int32_t* pos, int max_seq,
-                                          int max_len, float* part, int bw, hipStream_t st);
 
 extern "C" int64_t s2pk_attention_part_floats(int rows, int q_heads, int max_len) {
     const int nsplit = (max_len + AT_TILE * AT_WAVES - 1) / (AT_TILE * AT_WAVES);

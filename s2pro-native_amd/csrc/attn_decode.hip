@@ -36,9 +36,6 @@
 #include "attn_dev.h"
 #include "gemv_dev.h"
 
-extern "C" hipError_t s2p_attn_combine_launch(const float* part, uint16_t* out, int rows, int qh,
-                                              int nsplit, hipStream_t st);
-
 #define AD_WAVES 4
 #define AD_TILE 32 /* slots a wave takes at a time */
 
@@ -54,35 +51,11 @@ struct AdArgs {
     int rows, qh, kvh_n, max_seq, nsplit, split_pos;
 };
 
-#define AD_GLOBAL(T) const __attribute__((address_space(1))) T
 template <class T>
 S2P_DEV T ad_ld(const void* p) {
-    return *(AD_GLOBAL(T)*)p;
+    return *(GBL(T)*)p;
 }
 
-/* a uniform pointer in scalar registers, for loads of base + 32-bit offset */
-typedef AD_GLOBAL(char) * AdPtr;
-S2P_DEV AdPtr ad_base(const void* p, uint64_t off) {
-    const uint64_t v = (uint64_t)p + off;
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-    return (AdPtr)(((uint64_t)hi << 32) | lo);
-}
-template <class T, bool NT = false>
-S2P_DEV T ad_at(AdPtr p, uint32_t off) {
-    if constexpr (NT) return __builtin_nontemporal_load((AD_GLOBAL(T)*)(p + off));
-    else return *(AD_GLOBAL(T)*)(p + off);
-}
-
-/* 4 signed bytes -> 4 bf16 (exact) */
-S2P_DEV s2p_u32x2 ad_deq8(uint32_t d) {
-    const uint32_t f0 = __float_as_uint((float)(int8_t)(d & 0xFFu));
-    const uint32_t f1 = __float_as_uint((float)(int8_t)((d >> 8) & 0xFFu));
-    const uint32_t f2 = __float_as_uint((float)(int8_t)((d >> 16) & 0xFFu));
-    const uint32_t f3 = __float_as_uint((float)(int8_t)(d >> 24));
-    return (s2p_u32x2){__builtin_amdgcn_perm(f1, f0, 0x07060302u),
-                       __builtin_amdgcn_perm(f3, f2, 0x07060302u)};
-}
 /* a.hi half wave <-> b.lo; odd 16-lane rows of a <-> even rows of b */
 S2P_DEV void ad_swap32(uint32_t& a, uint32_t& b) {
     auto s = __builtin_amdgcn_permlane32_swap(a, b, false, false);
@@ -145,9 +118,9 @@ __global__ __launch_bounds__(64 * AD_WAVES) __attribute__((amdgpu_waves_per_eu(B
         return;
     }
     const uint64_t plane = (uint64_t)kvh * a.max_seq;
-    const AdPtr kb = ad_base(a.kcs[row], plane * EL), vb = ad_base(a.vcs[row], plane * EL);
-    const AdPtr ksb = BW == 16 ? kb : ad_base(a.kss[row], plane * 8);
-    const AdPtr vsb = BW == 16 ? vb : ad_base(a.vss[row], plane * 8);
+    const GblPtr kb = gbl_base(a.kcs[row], plane * EL), vb = gbl_base(a.vcs[row], plane * EL);
+    const GblPtr ksb = BW == 16 ? kb : gbl_base(a.kss[row], plane * 8);
+    const GblPtr vsb = BW == 16 ? vb : gbl_base(a.vss[row], plane * 8);
 
     auto load = [&](Tile& t, int tb) __attribute__((always_inline)) {
         const uint32_t last = (uint32_t)p_end - 1;
@@ -156,11 +129,11 @@ __global__ __launch_bounds__(64 * AD_WAVES) __attribute__((amdgpu_waves_per_eu(B
             const uint32_t slot = min((uint32_t)(tb + 16 * h + r), last);
 #pragma unroll
             for (int i = 0; i < Tile::NK; i++)
-                t.k[h][i] = ad_at<s2p_u32x4, BW == 16>(kb + 64 * i, slot * EL + 16u * q);
+                t.k[h][i] = gbl_at<s2p_u32x4, BW == 16>(kb + 64 * i, slot * EL + 16u * q);
             if constexpr (BW != 16) { /* the lane's four slots of the scores */
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    t.ks[h][i] = ad_at<s2p_u32x2>(
+                    t.ks[h][i] = gbl_at<s2p_u32x2>(
                         ksb, min((uint32_t)(tb + 16 * h + 4 * q + i), last) * 8u);
             }
         }
@@ -168,16 +141,16 @@ __global__ __launch_bounds__(64 * AD_WAVES) __attribute__((amdgpu_waves_per_eu(B
         for (int i = 0; i < Tile::NI; i++) {
             const uint32_t slot = min((uint32_t)(tb + i * Tile::NS + lane / LPS), last);
             if constexpr (BW == 4) {
-                const s2p_u32x2 w = ad_at<s2p_u32x2>(vb, slot * EL + 8u * (lane % LPS));
+                const s2p_u32x2 w = gbl_at<s2p_u32x2>(vb, slot * EL + 8u * (lane % LPS));
                 t.v[i][0] = w.x;
                 t.v[i][1] = w.y;
             } else {
-                const s2p_u32x4 w = ad_at<s2p_u32x4, BW == 16>(vb, slot * EL + 16u * (lane % LPS));
+                const s2p_u32x4 w = gbl_at<s2p_u32x4, BW == 16>(vb, slot * EL + 16u * (lane % LPS));
 #pragma unroll
                 for (int d = 0; d < 4; d++) t.v[i][d] = w[d];
             }
             if constexpr (BW != 16)
-                t.vs[i] = ad_at<uint16_t>(vsb, slot * 8u + 2u * ((lane % LPS) >> 1));
+                t.vs[i] = gbl_at<uint16_t>(vsb, slot * 8u + 2u * ((lane % LPS) >> 1));
         }
     };
 
@@ -193,10 +166,7 @@ __global__ __launch_bounds__(64 * AD_WAVES) __attribute__((amdgpu_waves_per_eu(B
             const int d = BW == 8 ? 32 * g + 16 * (q & 1) + 8 * (q >> 1) : 32 * g + 8 * q;
             s2p_u32x4 w = ad_ld<s2p_u32x4>(qr + d);
             if (BW == 4) /* the k-slot order of deq_int4 */
-                w = (s2p_u32x4){__builtin_amdgcn_perm(w.z, w.x, 0x05040100u),
-                                __builtin_amdgcn_perm(w.z, w.x, 0x07060302u),
-                                __builtin_amdgcn_perm(w.w, w.y, 0x05040100u),
-                                __builtin_amdgcn_perm(w.w, w.y, 0x07060302u)};
+                w = int4_order(w);
             qb[g] = r < 4 ? w : (s2p_u32x4){0u, 0u, 0u, 0u};
         }
     }
@@ -249,7 +219,7 @@ __global__ __launch_bounds__(64 * AD_WAVES) __attribute__((amdgpu_waves_per_eu(B
                 for (int g = 0; g < 4; g++) {
                     s2p_f32x4 raw;
                     if constexpr (BW == 8) {
-                        const s2p_u32x2 lo = ad_deq8(kd[g][0]), hi = ad_deq8(kd[g][1]);
+                        const s2p_u32x2 lo = deq_s8(kd[g][0]), hi = deq_s8(kd[g][1]);
                         raw = mfma16x16x32((s2p_u32x4){lo.x, lo.y, hi.x, hi.y}, qb[g],
                                            (s2p_f32x4){0.f, 0.f, 0.f, 0.f});
                     } else {
@@ -416,8 +386,6 @@ static int ad_rounds(int pairs, int units, bool bf16) {
     return best;
 }
 
-/* bw 16, 8 or 4; q_heads == 4 kv_heads.  part holds at least
- * ceil(max_len / 128) splits a (row, head); kss / vss: f16 scales (bw 8, 4) */
 extern "C" hipError_t s2p_attn_dec_launch(const uint16_t* q, const void* const* kcs,
                                           const void* const* vcs, const uint16_t* const* kss,
                                           const uint16_t* const* vss, uint16_t* out, int rows,

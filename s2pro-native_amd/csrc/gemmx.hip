@@ -22,7 +22,8 @@
  *   - neither goes through LDS, so waves run without barriers until their
  *     partial tiles meet there, where one thread per four outputs sums the K
  *     slices in order (deterministic).  K advances in chunks of 128, operands
- *     one chunk ahead.
+ *     one chunk ahead.  Up to 39 of the tiles' scalar bases and trip counts sit
+ *     in lanes of a vector register (INT4, T = 2, MTW = 4); nothing is in scratch.
  * INT4 weights become 1.5 + w / 16 (exact), the bias -1.5 sum x of a group is
  * an MFMA against a constant and the C operand of the group's products. */
 #include <hip/hip_runtime.h>
@@ -49,21 +50,6 @@ struct GmxArgs {
     int splits, np;    /* K splits over workgroups; columns of a partial row */
 };
 
-#define GX_GLOBAL(T) const __attribute__((address_space(1))) T
-typedef GX_GLOBAL(char) * GxPtr;
-/* scalar base (the compiler keeps products of uniform numbers in the vector
- * unit), so that a load is base + 32-bit lane offset + constant */
-S2P_DEV GxPtr gx_base(const void* p, uint64_t off) {
-    const uint64_t v = (uint64_t)p + off;
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-    return (GxPtr)(((uint64_t)hi << 32) | lo);
-}
-template <class T>
-S2P_DEV T gx_at(GxPtr base, uint32_t off) {
-    return *(GX_GLOBAL(T)*)(base + off);
-}
-
 /* bytes of a weight row per chunk, and 16-byte loads of it */
 static __host__ __device__ constexpr int gx_cb(int wfmt) {
     return wfmt == GEMV_W_INT4 ? 64 : wfmt == GEMV_W_INT8 ? 128 : 256;
@@ -77,23 +63,6 @@ struct GxW<GEMV_W_INT4> {
     s2p_u32x4 w[1];
     s2p_u32x2 s; /* the chunk's four f16 group scales of the lane's row */
 };
-
-/* INT4 k-slot order of deq_int4 (0,4 1,5 2,6 3,7) */
-S2P_DEV s2p_u32x4 gx_order(s2p_u32x4 v) {
-    return (s2p_u32x4){__builtin_amdgcn_perm(v.z, v.x, 0x05040100u),
-                       __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
-                       __builtin_amdgcn_perm(v.w, v.y, 0x05040100u),
-                       __builtin_amdgcn_perm(v.w, v.y, 0x07060302u)};
-}
-/* 4 signed bytes -> 4 bf16 (exact) */
-S2P_DEV s2p_u32x2 gx_deq8(uint32_t d) {
-    const uint32_t f0 = __float_as_uint((float)(int8_t)(d & 0xFFu));
-    const uint32_t f1 = __float_as_uint((float)(int8_t)((d >> 8) & 0xFFu));
-    const uint32_t f2 = __float_as_uint((float)(int8_t)((d >> 16) & 0xFFu));
-    const uint32_t f3 = __float_as_uint((float)(int8_t)(d >> 24));
-    return (s2p_u32x2){__builtin_amdgcn_perm(f1, f0, 0x07060302u),
-                       __builtin_amdgcn_perm(f3, f2, 0x07060302u)};
-}
 
 /* every argument in one round of scalar loads */
 S2P_DEV void gx_args(const GmxArgs& a) {
@@ -125,16 +94,16 @@ __global__ __launch_bounds__(64 * GX_WAVES) void k_gmx(GmxArgs a) {
 
     /* activation operands: tile c of this wave (past the last: it again, its
      * outputs are dropped), 4 KB a chunk and tile */
-    GxPtr xb[MTW];
+    GblPtr xb[MTW];
 #pragma unroll
     for (int c = 0; c < MTW; c++)
-        xb[c] = gx_base(a.x, ((uint64_t)c0 * a.mt + min(mg * MTW + c, a.mt - 1)) * 4096u);
+        xb[c] = gbl_base(a.x, ((uint64_t)c0 * a.mt + min(mg * MTW + c, a.mt - 1)) * 4096u);
     const uint32_t xs = (uint32_t)a.mt * 4096u, xl = 16u * lane;
 
     for (int g = blockIdx.x; g < a.groups; g += gridDim.x) {
         /* tiles: scalar base of the first row, lane offset of row r (past the
          * end: the last row again) */
-        GxPtr wb[T], sb[T];
+        GblPtr wb[T], sb[T];
         uint32_t wl[T], sl[T];
 #pragma unroll
         for (int t = 0; t < T; t++) {
@@ -142,10 +111,10 @@ __global__ __launch_bounds__(64 * GX_WAVES) void k_gmx(GmxArgs a) {
             const int n0 = min(ot * a.rpt, F - 1);
             const uint32_t rl = (uint32_t)min(r, min(a.rpt, F - n0) - 1);
             const uint64_t row0 = (uint64_t)(n0 + (sw && rg ? F : 0));
-            wb[t] = gx_base(a.w, row0 * rb + (uint64_t)c0 * gx_cb(WFMT));
+            wb[t] = gbl_base(a.w, row0 * rb + (uint64_t)c0 * gx_cb(WFMT));
             wl[t] = rl * rb + 16u * q;
             if constexpr (WFMT == GEMV_W_INT4) {
-                sb[t] = gx_base(a.s, row0 * (uint32_t)(a.K >> 4) + (uint64_t)c0 * 8);
+                sb[t] = gbl_base(a.s, row0 * (uint32_t)(a.K >> 4) + (uint64_t)c0 * 8);
                 sl[t] = rl * (uint32_t)(a.K >> 4);
             }
         }
@@ -157,15 +126,15 @@ __global__ __launch_bounds__(64 * GX_WAVES) void k_gmx(GmxArgs a) {
             for (int t = 0; t < T; t++) {
 #pragma unroll
                 for (int l = 0; l < NL; l++)
-                    w[t].w[l] = gx_at<s2p_u32x4>(wb[t] + ck * gx_cb(WFMT) + l * 64, wl[t]);
+                    w[t].w[l] = gbl_at<s2p_u32x4>(wb[t] + ck * gx_cb(WFMT) + l * 64, wl[t]);
                 if constexpr (WFMT == GEMV_W_INT4)
-                    w[t].s = gx_at<s2p_u32x2>(sb[t] + ck * 8, sl[t]);
+                    w[t].s = gbl_at<s2p_u32x2>(sb[t] + ck * 8, sl[t]);
             }
 #pragma unroll
             for (int c = 0; c < MTW; c++)
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    x[c][i] = gx_at<s2p_u32x4>(xb[c] + (size_t)ck * xs + i * 1024, xl);
+                    x[c][i] = gbl_at<s2p_u32x4>(xb[c] + (size_t)ck * xs + i * 1024, xl);
         };
         s2p_f32x4 acc[T][MTW];
 #pragma unroll
@@ -214,8 +183,8 @@ __global__ __launch_bounds__(64 * GX_WAVES) void k_gmx(GmxArgs a) {
                     for (int t = 0; t < T; t++) {
                         s2p_u32x4 wv;
                         if constexpr (WFMT == GEMV_W_INT8) {
-                            const s2p_u32x2 lo = gx_deq8(w[t].w[i >> 1][2 * (i & 1)]);
-                            const s2p_u32x2 hi = gx_deq8(w[t].w[i >> 1][2 * (i & 1) + 1]);
+                            const s2p_u32x2 lo = deq_s8(w[t].w[i >> 1][2 * (i & 1)]);
+                            const s2p_u32x2 hi = deq_s8(w[t].w[i >> 1][2 * (i & 1) + 1]);
                             wv = (s2p_u32x4){lo.x, lo.y, hi.x, hi.y};
                         } else {
                             wv = w[t].w[i];
@@ -429,7 +398,7 @@ __global__ __launch_bounds__(512) void k_gmx_pack(const uint16_t* __restrict__ x
                        ((uint32_t)f2bf(__fmul_rn(__fmul_rn(bf2f_hi(v[d]), inv), bf2f_hi(wv[d])))
                         << 16);
         }
-        if constexpr (WFMT == GEMV_W_INT4) v = gx_order(v);
+        if constexpr (WFMT == GEMV_W_INT4) v = int4_order(v);
         *(s2p_u32x4*)(xp + (((size_t)ck * mt + ct) * 256 + (it & 255)) * 8) = v;
     }
 }

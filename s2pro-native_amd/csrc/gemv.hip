@@ -1,14 +1,20 @@
-/* s2pro MI355X — weight-only INT4 / INT8 GEMV engine for decode / verify M.
+/* s2pro MI355X — dispatch of the weight GEMVs / GEMMs, and the two staged
+ * engines: activations in LDS, weights through the INT4 / INT8 / bf16 MFMA tile.
  *
  * Replaces the reference's packed-INT4 and per-channel INT8 GEMVs
  * (src/sched/int8_gemv.cu:60-104, 279-324, 836-902, 964-986) and its M > 16
- * dequant + cuBLAS / WMMA paths (gemm.c:444-490, int8_gemv.cu:535-618) with
- * one MI355X kernel.
+ * dequant + cuBLAS / WMMA paths (gemm.c:444-490, int8_gemv.cu:535-618).
+ * s2p_gemv_launch takes, in this order: M <= 16 k_gvr / k_gvs (gemvr.hip), M > 16
+ * k_gmx (gemmx.hip) and, INT4 at M <= 96, k_gemm4 (gemm4.hip); what these leave
+ * (other K, shapes where one below is faster) and every plan over quantised
+ * caches that is not k_gemm4's goes to
+ *   k_gemv3  whole-K workgroups of up to 16 waves, M <= 16, or 8 waves, M <= 32
+ *            (not INT4), where the activations fit in LDS;
+ *   k_gemv   split K, any M <= 128 (not bf16).
  *
- * Work decomposition.  The N output rows form 64-row blocks, K forms S
- * splits.  The grid is (P, S): workgroup (p, s) stages the activations of
- * split s in LDS once and then streams the weights of row blocks p, p+P,
- * p+2P, ...; P is sized so the grid is about one resident round of
+ * k_gemv: the N output rows form 64-row blocks, K forms S splits.  The grid is
+ * (P, S): workgroup (p, s) stages the activations of split s in LDS once and
+ * then streams the weights of row blocks p, p+P, p+2P, ...; P is sized so the grid is about one resident round of
  * workgroups, so the staging is paid once per workgroup, not once per block.
  * Wave w owns rows 16w..16w+15 of the current block and runs its own weight
  * stream, double buffered (the next chunk's 16-byte loads are in flight
@@ -34,7 +40,7 @@
  * bf16; result = s_n (acc - 128 sum_k x_k).
  *
  * Staging applies the consuming layer's RMSNorm (row inverse RMS from the
- * producer epilogue's per-64-column sums of squares) with the rule's
+ * producer epilogue's per-16-column sums of squares) with the rule's
  * roundings.  Epilogues: bf16 store; residual add y = bf16(y + bf16(acc))
  * (kernels.cu:1242-1247) with sums of squares for the next RMSNorm; or
  * SwiGLU, where a block holds 32 gate rows and the 32 matching up rows and
@@ -66,8 +72,8 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void k_gemv3(GemvArgs a) {
                  "s"(a.K), "s"(a.gps), "s"(a.ks), "s"(a.rt), "s"(a.xmode), "s"(a.epi),
                  "s"(a.ssq_in_blocks), "s"(a.norm_eps), "s"(gridDim.x));
     GvBuf b0, b1;
-    gv3_block<WFMT, MT, false, false, false, false>(a, blockIdx.x, gridDim.x,
-                                                   (LDS(unsigned char)*)smem3, a.y, b0, b1);
+    gv3_block<WFMT, MT>(a, blockIdx.x, gridDim.x,
+                        (LDS(unsigned char)*)smem3, a.y, b0, b1);
 }
 
 template <int WFMT, int MT, bool WIN1>

@@ -71,6 +71,42 @@ S2P_DEV s2p_u32x2 deq_int8(uint32_t d) {
     return r;
 }
 
+/* Global loads as scalar base + 32-bit lane offset + constant: one address
+ * register a lane, not a 64-bit pair per load.  The base goes through
+ * readfirstlane: left to itself the compiler multiplies uniform row numbers in
+ * the vector unit and keeps the sums there */
+#define GBL(T) const __attribute__((address_space(1))) T
+typedef GBL(char) * GblPtr;
+S2P_DEV GblPtr gbl_base(const void* p, uint64_t off) {
+    const uint64_t v = (uint64_t)p + off;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (GblPtr)(((uint64_t)hi << 32) | lo);
+}
+/* NT: nontemporal (past the caches) */
+template <class T, bool NT = false>
+S2P_DEV T gbl_at(GblPtr base, uint32_t off) {
+    if constexpr (NT) return __builtin_nontemporal_load((GBL(T)*)(base + off));
+    else return *(GBL(T)*)(base + off);
+}
+
+/* 8 bf16 in the k-slot order of deq_int4 (0,4 1,5 2,6 3,7) */
+S2P_DEV s2p_u32x4 int4_order(s2p_u32x4 v) {
+    return (s2p_u32x4){__builtin_amdgcn_perm(v.z, v.x, 0x05040100u),
+                       __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
+                       __builtin_amdgcn_perm(v.w, v.y, 0x05040100u),
+                       __builtin_amdgcn_perm(v.w, v.y, 0x07060302u)};
+}
+/* 4 signed bytes -> 4 bf16 (exact) */
+S2P_DEV s2p_u32x2 deq_s8(uint32_t d) {
+    const uint32_t f0 = __float_as_uint((float)(int8_t)(d & 0xFFu));
+    const uint32_t f1 = __float_as_uint((float)(int8_t)((d >> 8) & 0xFFu));
+    const uint32_t f2 = __float_as_uint((float)(int8_t)((d >> 16) & 0xFFu));
+    const uint32_t f3 = __float_as_uint((float)(int8_t)(d >> 24));
+    return (s2p_u32x2){__builtin_amdgcn_perm(f1, f0, 0x07060302u),
+                       __builtin_amdgcn_perm(f3, f2, 0x07060302u)};
+}
+
 /* silu(g) * u with the two bf16 roundings of kernels.cu:1216-1229; exp is
  * the rule's s2p_expf so the value matches the host oracle bit for bit. */
 S2P_DEV uint16_t silu_mul_bf16(uint16_t g16, uint16_t u16) {
@@ -997,7 +1033,6 @@ struct Gv3Pre {
     float ssq[3];
 };
 
-template <bool COH>
 S2P_DEV void gv3_pre_issue(const GemvArgs& a, Gv3Pre& pre, bool stager, int wave, int lane,
                            int gb, int gn) {
     const int M = a.M;
@@ -1006,21 +1041,15 @@ S2P_DEV void gv3_pre_issue(const GemvArgs& a, Gv3Pre& pre, bool stager, int wave
 #pragma unroll
         for (int i = 0; i < 3; i++)
             if (lane + 64 * i < a.ssq_in_blocks)
-                pre.ssq[i] = ld_actf<COH>(a.ssq_in + (size_t)(lane + 64 * i) * GEMV_MAX_M + wave);
+                pre.ssq[i] = a.ssq_in[(size_t)(lane + 64 * i) * GEMV_MAX_M + wave];
     }
     if (stager && lane < gn * 4) {
         const int k = gb * 32 + lane * 8;
 #pragma unroll
         for (int m = 0; m < 8; m++)
-            if (m < M) pre.raw[m] = ld_act128<COH>(a.x + (size_t)m * a.ldx + k);
+            if (m < M) pre.raw[m] = ld_act128<false>(a.x + (size_t)m * a.ldx + k);
         if (norm) pre.wn4 = *(const s2p_u32x4*)(a.norm_w + k);
     }
-}
-
-template <bool COH>
-S2P_DEV void st_act16(uint16_t* p, uint16_t v) {
-    if constexpr (COH) coh_st16(p, v);
-    else *p = v;
 }
 
 /* Work geometry of workgroup p of P and of one of its waves. */
@@ -1061,51 +1090,23 @@ S2P_DEV int gv3_wrow(const GemvArgs& a, const Gv3Geo& g, int tg, int r) {
     return min(base + r, a.N - 1);
 }
 
-/* INT4 at one column tile runs the transposed tile (gv_compute TR), except
- * in the persistent kernel (NOTR), whose register budget the untransposed
- * tile fits, and in layer launches shaped like it (the test hook that
- * compares the two) */
-static __host__ __device__ constexpr bool gv3_tr(int wfmt, int mt, bool notr) {
-    return wfmt == GEMV_W_INT4 && mt == 1 && !notr;
+/* INT4 at one column tile runs the transposed tile (gv_compute TR) */
+static __host__ __device__ constexpr bool gv3_tr(int wfmt, int mt) {
+    return wfmt == GEMV_W_INT4 && mt == 1;
 }
 
 /* chunk t of the wave's flattened (tile group, chunk) stream */
-template <int WFMT, int MT, bool NOTR>
+template <int WFMT, int MT>
 S2P_DEV void gv3_load(GvBuf& B, const GemvArgs& a, const Gv3Geo& g, int p, int P, int t) {
     constexpr int CHG = gv_chg(WFMT);
     const int lane = threadIdx.x & 63;
     const int it = g.nch == 1 ? t : t / g.nch, c = t - it * g.nch;
-    gv_load<WFMT, gv3_tr(WFMT, MT, NOTR)>(B, a, gv3_wrow(a, g, p + it * P, lane & 15), g.gb + c * CHG,
+    gv_load<WFMT, gv3_tr(WFMT, MT)>(B, a, gv3_wrow(a, g, p + it * P, lane & 15), g.gb + c * CHG,
                   min(CHG, g.gn - c * CHG), lane >> 4);
 }
 
-/* The first weight chunk of workgroup p, issued ahead (the persistent kernel
- * issues it before the barrier that precedes the GEMV). */
-template <int WFMT, int MT = 1>
-S2P_DEV void gv3_prefetch(const GemvArgs& a, int p, int P, GvBuf& b0, GvBuf& b1) {
-    const Gv3Geo g = gv3_geo<WFMT>(a, p, P, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
-    /* both buffers defined on every path: their old contents are dead */
-    if (g.T > 0) {
-        gv3_load<WFMT, MT, true>(b0, a, g, p, P, 0);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; i++) b0.w[i] = 0u;
-        b0.s = (s2p_u32x2){0u, 0u};
-    }
-    if (g.T > 1) {
-        gv3_load<WFMT, MT, true>(b1, a, g, p, P, 1);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; i++) b1.w[i] = 0u;
-        b1.s = (s2p_u32x2){0u, 0u};
-    }
-}
-
-/* PRE: b0 and b1 already hold (or are loading) the first two chunks
- * (gv3_prefetch). */
-/* COH: activation loads bypass the L2 (their producer ran in this launch
- * and the L2 was not invalidated since); WT: outputs written through. */
-template <int WFMT, int MT, bool COH, bool PRE = false, bool WT = COH, bool NOTR = PRE>
+/* workgroup p of P */
+template <int WFMT, int MT>
 __device__ void gv3_block(const GemvArgs& a, int p, int P, LDS(unsigned char)* smem,
                           uint16_t* Y, GvBuf& b0, GvBuf& b1) {
 #pragma clang fp contract(off)
@@ -1152,12 +1153,12 @@ __device__ void gv3_block(const GemvArgs& a, int p, int P, LDS(unsigned char)* s
 
     const int nch = geo.nch, T = geo.T;
     auto load_t = [&](GvBuf& B, int t) __attribute__((always_inline)) {
-        gv3_load<WFMT, MT, NOTR>(B, a, geo, p, P, t);
+        gv3_load<WFMT, MT>(B, a, geo, p, P, t);
     };
 
     Gv3Pre pre;
-    gv3_pre_issue<COH>(a, pre, geo.j == 0, wave, lane, gb, gn);
-    if constexpr (!PRE) load_t(b0, 0); /* in flight during the staging */
+    gv3_pre_issue(a, pre, geo.j == 0, wave, lane, gb, gn);
+    load_t(b0, 0); /* in flight during the staging */
     if (a.xmode == GEMV_X_NORM) {
         /* inverse RMS per row: lanes take the producer's blocks, fixed-order
          * wave reduction */
@@ -1169,7 +1170,7 @@ __device__ void gv3_block(const GemvArgs& a, int p, int P, LDS(unsigned char)* s
                     if (lane + 64 * i < a.ssq_in_blocks) s += pre.ssq[i];
             } else {
                 for (int b = lane; b < a.ssq_in_blocks; b += 64)
-                    s += ld_actf<COH>(a.ssq_in + (size_t)b * GEMV_MAX_M + m);
+                    s += a.ssq_in[(size_t)b * GEMV_MAX_M + m];
             }
             s = wave_sum_down(s);
             if (lane == 0) L.inv[m] = rsqrt_rule(s / (float)a.K + a.norm_eps);
@@ -1198,7 +1199,7 @@ __device__ void gv3_block(const GemvArgs& a, int p, int P, LDS(unsigned char)* s
 #pragma unroll
                 for (int jj = 0; jj < 4; jj++)
                     raw[jj] = (valid && m0 + jj < M)
-                                  ? ld_act128<COH>(a.x + (size_t)(m0 + jj) * a.ldx + k)
+                                  ? ld_act128<false>(a.x + (size_t)(m0 + jj) * a.ldx + k)
                                   : (s2p_u32x4){0u, 0u, 0u, 0u};
 #pragma unroll
                 for (int jj = 0; jj < 4; jj++)
@@ -1250,178 +1251,103 @@ __device__ void gv3_block(const GemvArgs& a, int p, int P, LDS(unsigned char)* s
         if (it == 0) stamp(3);
         __syncthreads();
         if (it == 0) stamp(4);
-        if constexpr (NOTR) {
-            /* output (row rho of unit u, column m): element rho % 4 of lane
-             * (rho / 4) * 16 + m % 16, column tile m / 16, of the unit's waves */
+        /* Unit u (a 16-row output tile; SWIGLU: its gate and up tiles) is
+         * reduced by its own waves, lane-locally: a lane sums its elements
+         * over the ks K-slice partials in slice order (deterministic), then
+         * runs the epilogue.  Element i of lane (q, r) in column tile t is
+         * (m, n) = (16t + 4q + i, r) for the transposed INT4 tile, and
+         * (16t + r, 4q + i) otherwise.  Transposed: element i is handled by
+         * the unit's slice wave i % ks (the per-column sums of squares are
+         * per element); otherwise slice wave 0 takes all four. */
+        constexpr bool TRN = gv3_tr(WFMT, MT);
+        const int u = geo.j, sl0 = geo.sp;
+        const int tile = (p + it * P) * units + u;
+        if (u < units && tile < tiles && (TRN || sl0 == 0)) { /* uniform */
+            const int n0 = tile * 16;
             const LDS(float)* rf = (const LDS(float)*)rb;
-            const int g = p + it * P;
-            auto tsum = [&](int jw, int rho, int m) __attribute__((always_inline)) {
-                const int src = ((m >> 4) * 64 + (rho >> 2) * 16 + (m & 15)) * 4 + (rho & 3);
-                float v = 0.f;
-                for (int s = 0; s < ks; s++) v += rf[(size_t)(jw * ks + s) * MT * 256 + src];
-                return v;
-            };
-            for (int u = 0; u < units; u++)
-            for (int base = 0; base < M * 16; base += nw * 64) {
-                const int idx = base + tid;
-                const int rho = idx & 15, m = idx >> 4;
-                const int tile = g * units + u;
-                const int n = tile * 16 + rho;
-                const bool ok = m < M && tile < tiles;
-                if (swiglu) {
-                    if (ok) {
-                        float gv = tsum(u, rho, m), uv = tsum(units + u, rho, m);
-                        if (WFMT == GEMV_W_INT8) {
-                            gv *= ((const float*)a.s)[n];
-                            uv *= ((const float*)a.s)[F + n];
-                        }
-                        st_act16<WT>(Y + (size_t)m * a.ldy + n, silu_mul_bf16(f2bf(gv), f2bf(uv)));
-                    }
-                    continue;
-                }
-                float ssq = 0.f;
-                if (ok && n < a.N) {
-                    float v = tsum(u, rho, m);
-                    if (WFMT == GEMV_W_INT8) v *= ((const float*)a.s)[n];
-                    const uint16_t yb = f2bf(v);
-                    uint16_t* yp = Y + (size_t)m * a.ldy + n;
-                    if (a.epi == GEMV_EPI_RESID) {
-                        const uint16_t xo = f2bf(__fadd_rn(bf2f(ld_act16<COH>(yp)), bf2f(yb)));
-                        st_act16<WT>(yp, xo);
-                        const float xv = bf2f(xo);
-                        ssq = xv * xv;
-                    } else {
-                        st_act16<WT>(yp, yb);
-                    }
-                }
-                if (a.epi == GEMV_EPI_RESID && a.ssq_out) {
-                    const float tot = sum_lanes16(ssq); /* the 16 rows of (tile, m) */
-                    if (rho == 0 && ok) coh_stf(a.ssq_out + (size_t)tile * GEMV_MAX_M + m, tot);
-                }
-            }
-        } else {
-            /* Unit u (a 16-row output tile; SWIGLU: its gate and up tiles) is
-             * reduced by its own waves, lane-locally: a lane sums its elements
-             * over the ks K-slice partials in slice order (deterministic), then
-             * runs the epilogue.  Element i of lane (q, r) in column tile t is
-             * (m, n) = (16t + 4q + i, r) for the transposed INT4 tile, and
-             * (16t + r, 4q + i) otherwise.  Transposed: element i is handled by
-             * the unit's slice wave i % ks (the per-column sums of squares are
-             * per element); otherwise slice wave 0 takes all four. */
-            constexpr bool TRN = gv3_tr(WFMT, MT, NOTR);
-            const int u = geo.j, sl0 = geo.sp;
-            const int tile = (p + it * P) * units + u;
-            if (u < units && tile < tiles && (TRN || sl0 == 0)) { /* uniform */
-                const int n0 = tile * 16;
-                const LDS(float)* rf = (const LDS(float)*)rb;
-    #pragma unroll 1
-                for (int t = 0; t < MT; t++) {
-                    float sq4 = 0.f;
-    #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        if (TRN && i % ks != sl0) continue; /* uniform */
-                        float v = 0.f, w = 0.f;
+#pragma unroll 1
+            for (int t = 0; t < MT; t++) {
+                float sq4 = 0.f;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (TRN && i % ks != sl0) continue; /* uniform */
+                    float v = 0.f, w = 0.f;
+                    for (int sl = 0; sl < ks; sl++)
+                        v += rf[(((u * ks + sl) * MT + t) * 64 + lane) * 4 + i];
+                    if (swiglu)
                         for (int sl = 0; sl < ks; sl++)
-                            v += rf[(((u * ks + sl) * MT + t) * 64 + lane) * 4 + i];
-                        if (swiglu)
-                            for (int sl = 0; sl < ks; sl++)
-                                w += rf[((((units + u) * ks + sl) * MT + t) * 64 + lane) * 4 + i];
-                        const int m = TRN ? t * 16 + 4 * q + i : t * 16 + r;
-                        const int n = n0 + (TRN ? r : 4 * q + i);
-                        const bool ok = m < M;
-                        if (swiglu) {
-                            if (ok) {
-                                float gv = v, uv = w;
-                                if (WFMT == GEMV_W_INT8) {
-                                    gv *= ((const float*)a.s)[n];
-                                    uv *= ((const float*)a.s)[F + n];
-                                }
-                                st_act16<WT>(Y + (size_t)m * a.ldy + n,
-                                             silu_mul_bf16(f2bf(gv), f2bf(uv)));
+                            w += rf[((((units + u) * ks + sl) * MT + t) * 64 + lane) * 4 + i];
+                    const int m = TRN ? t * 16 + 4 * q + i : t * 16 + r;
+                    const int n = n0 + (TRN ? r : 4 * q + i);
+                    const bool ok = m < M;
+                    if (swiglu) {
+                        if (ok) {
+                            float gv = v, uv = w;
+                            if (WFMT == GEMV_W_INT8) {
+                                gv *= ((const float*)a.s)[n];
+                                uv *= ((const float*)a.s)[F + n];
                             }
-                            continue;
+                            Y[(size_t)m * a.ldy + n] = silu_mul_bf16(f2bf(gv), f2bf(uv));
                         }
-                        float sq = 0.f;
-                        if (ok && n < a.N) {
-                            if (WFMT == GEMV_W_INT8) v *= ((const float*)a.s)[n];
-                            const uint16_t yb = f2bf(v);
-                            uint16_t* yp = Y + (size_t)m * a.ldy + n;
-                            if (a.epi == GEMV_EPI_RESID) {
-                                const uint16_t xo = f2bf(__fadd_rn(bf2f(ld_act16<COH>(yp)), bf2f(yb)));
-                                st_act16<WT>(yp, xo);
-                                const float xv = bf2f(xo);
-                                sq = xv * xv;
-                            } else {
-                                st_act16<WT>(yp, yb);
-                            }
-                        }
-                        if (a.epi == GEMV_EPI_RESID && a.ssq_out) {
-                            if (TRN) {
-                                /* over the tile's 16 rows n = r of column m */
-                                const float tot = sum_lanes16(sq);
-                                if (r == 0 && ok)
-                                    coh_stf(a.ssq_out + (size_t)tile * GEMV_MAX_M + m, tot);
-                            } else {
-                                sq4 += sq;
-                            }
+                        continue;
+                    }
+                    float sq = 0.f;
+                    if (ok && n < a.N) {
+                        if (WFMT == GEMV_W_INT8) v *= ((const float*)a.s)[n];
+                        const uint16_t yb = f2bf(v);
+                        uint16_t* yp = Y + (size_t)m * a.ldy + n;
+                        if (a.epi == GEMV_EPI_RESID) {
+                            const uint16_t xo = f2bf(__fadd_rn(bf2f(*yp), bf2f(yb)));
+                            *yp = xo;
+                            const float xv = bf2f(xo);
+                            sq = xv * xv;
+                        } else {
+                            *yp = yb;
                         }
                     }
-                    if (!TRN && !swiglu && a.epi == GEMV_EPI_RESID && a.ssq_out) {
-                        float tot = sq4;
-                        tot += __shfl_xor(tot, 16, 64);
-                        tot += __shfl_xor(tot, 32, 64);
-                        const int m = t * 16 + r;
-                        if (q == 0 && m < M)
-                            coh_stf(a.ssq_out + (size_t)tile * GEMV_MAX_M + m, tot);
+                    if (a.epi == GEMV_EPI_RESID && a.ssq_out) {
+                        if (TRN) {
+                            /* over the tile's 16 rows n = r of column m */
+                            const float tot = sum_lanes16(sq);
+                            if (r == 0 && ok)
+                                coh_stf(a.ssq_out + (size_t)tile * GEMV_MAX_M + m, tot);
+                        } else {
+                            sq4 += sq;
+                        }
                     }
+                }
+                if (!TRN && !swiglu && a.epi == GEMV_EPI_RESID && a.ssq_out) {
+                    float tot = sq4;
+                    tot += __shfl_xor(tot, 16, 64);
+                    tot += __shfl_xor(tot, 32, 64);
+                    const int m = t * 16 + r;
+                    if (q == 0 && m < M)
+                        coh_stf(a.ssq_out + (size_t)tile * GEMV_MAX_M + m, tot);
                 }
             }
         }
     };
     auto step = [&](const GvBuf& B, int t) __attribute__((always_inline)) {
         const int it = nch == 1 ? t : t / nch, c = t - it * nch;
-        gv_compute<WFMT, MT, gv3_tr(WFMT, MT, NOTR)>(B, L, c * CHG, min(CHG, gn - c * CHG), M, 0, q, r, acc, corr);
+        gv_compute<WFMT, MT, gv3_tr(WFMT, MT)>(B, L, c * CHG, min(CHG, gn - c * CHG), M, 0, q, r, acc, corr);
         if (c == nch - 1) finish(it);
     };
     int t = 0;
-    if constexpr (!PRE) {
-        /* one chunk ahead: b1 is loaded while b0 is multiplied; every path
-         * into a step has the same loads outstanding, and no load is issued
-         * past the end */
-        for (; t + 2 < T; t += 2) {
-            load_t(b1, t + 1);
-            step(b0, t);
-            load_t(b0, t + 2);
-            step(b1, t + 1);
-        }
-        if (T - t == 2) {
-            load_t(b1, t + 1);
-            step(b0, t);
-            step(b1, t + 1);
-        } else {
-            step(b0, t);
-        }
-    } else {
-    /* b0 holds chunk t and b1 chunk t + 1 (both issued before the barrier):
-     * two chunks in flight, every load in the loop unconditional, no load
-     * issued past the end */
-    for (; t + 3 < T; t += 2) {
+    /* one chunk ahead: b1 is loaded while b0 is multiplied; every path
+     * into a step has the same loads outstanding, and no load is issued
+     * past the end */
+    for (; t + 2 < T; t += 2) {
+        load_t(b1, t + 1);
         step(b0, t);
         load_t(b0, t + 2);
         step(b1, t + 1);
-        load_t(b1, t + 3);
     }
-    if (T - t == 3) {
-        step(b0, t);
-        load_t(b0, t + 2);
-        step(b1, t + 1);
-        step(b0, t + 2);
-    } else if (T - t == 2) {
+    if (T - t == 2) {
+        load_t(b1, t + 1);
         step(b0, t);
         step(b1, t + 1);
     } else {
         step(b0, t);
-    }
     }
     if (probe) {
         vm_drain();

@@ -77,28 +77,11 @@ struct GvrUnit<GEMV_W_INT4, WIDE> {
     s2p_u32x4 s;
 };
 
-/* Loads as scalar base + 32-bit lane offset + constant: one address register
- * a lane, not a 64-bit pair per load.  The base goes through readfirstlane:
- * left to itself the compiler multiplies the uniform row number in the vector
- * unit and keeps the sum there */
-#define GR_GLOBAL(T) const __attribute__((address_space(1))) T
-typedef GR_GLOBAL(char) * GrPtr;
-S2P_DEV GrPtr gr_base(const void* p, uint64_t off) {
-    const uint64_t v = (uint64_t)p + off;
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-    return (GrPtr)(((uint64_t)hi << 32) | lo);
-}
-template <class T>
-S2P_DEV T gr_at(GrPtr base, uint32_t off) {
-    return *(GR_GLOBAL(T)*)(base + off);
-}
-
 /* a tile: scalar bases of its first row (at unit u0), and the lane's byte
  * offsets: weight rows (one a load) and the row of its INT4 scales */
 template <int WFMT, bool WIDE>
 struct GvrTile {
-    GrPtr w, s;
+    GblPtr w, s;
     uint32_t wl[WIDE ? 2 : 1], sl;
 };
 
@@ -107,8 +90,8 @@ template <int WFMT, bool WIDE>
 S2P_DEV void gr_load(GvrUnit<WFMT, WIDE>& b, const GvrTile<WFMT, WIDE>& t, int u) {
 #pragma unroll
     for (int i = 0; i < (WIDE ? 2 : 1); i++)
-        b.w[i] = __builtin_nontemporal_load((GR_GLOBAL(s2p_u32x4)*)(t.w + u * 128 + t.wl[i]));
-    if constexpr (WFMT == GEMV_W_INT4) b.s = gr_at<s2p_u32x4>(t.s + u * 16, t.sl);
+        b.w[i] = gbl_at<s2p_u32x4, true>(t.w + u * 128, t.wl[i]);
+    if constexpr (WFMT == GEMV_W_INT4) b.s = gbl_at<s2p_u32x4>(t.s + u * 16, t.sl);
 }
 
 /* activation operand j of unit u: the k values its MFMA pairs with the
@@ -123,32 +106,12 @@ S2P_DEV uint32_t gr_klane(int q, int hi) {
 /* WIDE: operands 0 .. NX / 2 - 1 go with the even chunks, the rest with the
  * odd; u: units past the base */
 template <int WFMT, bool WIDE>
-S2P_DEV s2p_u32x4 gr_ldx(GrPtr x, uint32_t xl, int u, int j) {
+S2P_DEV s2p_u32x4 gr_ldx(GblPtr x, uint32_t xl, int u, int j) {
     constexpr int H = gr_nx(WFMT, false), ODD = WFMT == GEMV_W_INT4 ? 64 : WFMT == GEMV_W_INT8 ? 32 : 16;
     const int jj = WIDE ? j % H : j, odd = WIDE ? j / H : 0;
-    return gr_at<s2p_u32x4>(
+    return gbl_at<s2p_u32x4>(
         x + u * (2 * gr_uk(WFMT)) + jj * (WFMT == GEMV_W_INT4 ? 128 : 16) + odd * ODD, xl);
 }
-/* INT4 k-slot order of deq_int4 (0,4 1,5 2,6 3,7) */
-template <int WFMT>
-S2P_DEV s2p_u32x4 gr_order(s2p_u32x4 v) {
-    if constexpr (WFMT != GEMV_W_INT4) return v;
-    return (s2p_u32x4){__builtin_amdgcn_perm(v.z, v.x, 0x05040100u),
-                       __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
-                       __builtin_amdgcn_perm(v.w, v.y, 0x05040100u),
-                       __builtin_amdgcn_perm(v.w, v.y, 0x07060302u)};
-}
-
-/* 4 signed bytes -> 4 bf16 (exact) */
-S2P_DEV s2p_u32x2 gr_deq8(uint32_t d) {
-    const uint32_t f0 = __float_as_uint((float)(int8_t)(d & 0xFFu));
-    const uint32_t f1 = __float_as_uint((float)(int8_t)((d >> 8) & 0xFFu));
-    const uint32_t f2 = __float_as_uint((float)(int8_t)((d >> 16) & 0xFFu));
-    const uint32_t f3 = __float_as_uint((float)(int8_t)(d >> 24));
-    return (s2p_u32x2){__builtin_amdgcn_perm(f1, f0, 0x07060302u),
-                       __builtin_amdgcn_perm(f3, f2, 0x07060302u)};
-}
-
 /* lanes r < 8 of a, lanes r >= 8 from lanes r - 8 of b; and lanes r < 8 from
  * lanes r + 8 of a, lanes r >= 8 of b (DPP row_ror:8 on half the banks) */
 S2P_DEV uint32_t gr_lo(uint32_t a, uint32_t b) {
@@ -178,7 +141,7 @@ S2P_DEV void gr_chunk(s2p_u32x4 w, const s2p_u32x4* x, const s2p_f32x4* cb, s2p_
             for (int i = 0; i < 4; i++) acc[i] = fmaf(sf, raw[i], acc[i]);
         }
     } else if constexpr (WFMT == GEMV_W_INT8) {
-        const s2p_u32x2 a0 = gr_deq8(w.x), a1 = gr_deq8(w.y), a2 = gr_deq8(w.z), a3 = gr_deq8(w.w);
+        const s2p_u32x2 a0 = deq_s8(w.x), a1 = deq_s8(w.y), a2 = deq_s8(w.z), a3 = deq_s8(w.w);
         acc = mfma16x16x32(x[0], (s2p_u32x4){a0.x, a0.y, a1.x, a1.y}, acc);
         acc = mfma16x16x32(x[1], (s2p_u32x4){a2.x, a2.y, a3.x, a3.y}, acc);
     } else {
@@ -243,12 +206,12 @@ S2P_DEV GvrTile<WFMT, WIDE> gr_tile(const GvrArgs& a, int g, int j, int ntp, int
                                                          : a.K * 2); /* bytes of a row */
     const uint32_t ch = 16u * (2 * q + (r >> 3));
     GvrTile<WFMT, WIDE> t;
-    t.w = gr_base(a.w, row0 * rb + (uint64_t)u0 * 128);
+    t.w = gbl_base(a.w, row0 * rb + (uint64_t)u0 * 128);
     t.wl[0] = (uint32_t)min(r & 7, last) * rb + ch;
     if constexpr (WIDE) t.wl[1] = (uint32_t)min(8 + (r & 7), last) * rb + ch;
     if constexpr (WFMT == GEMV_W_INT4) {
         const uint32_t sb = (uint32_t)(a.K >> 4);
-        t.s = gr_base(a.s, row0 * sb + (uint64_t)u0 * 16);
+        t.s = gbl_base(a.s, row0 * sb + (uint64_t)u0 * 16);
         t.sl = (uint32_t)min(WIDE ? r : (r & 7), last) * sb;
     }
     return t;
@@ -391,7 +354,7 @@ __global__ __launch_bounds__(64 * NW) void k_gvr(GvrArgs a) {
 #pragma unroll
         for (int j = 0; j < NX; j++) x[u][j] = (s2p_u32x4){0u, 0u, 0u, 0u};
     if (mrow < a.M) {
-        const GrPtr xb = gr_base(a.x, (uint64_t)u0 * (2 * gr_uk(WFMT)));
+        const GblPtr xb = gbl_base(a.x, (uint64_t)u0 * (2 * gr_uk(WFMT)));
         const uint32_t xl = (uint32_t)mrow * (uint32_t)a.ldx * 2u + kl;
 #pragma unroll
         for (int u = 0; u < U; u++)
@@ -399,7 +362,7 @@ __global__ __launch_bounds__(64 * NW) void k_gvr(GvrArgs a) {
             for (int j = 0; j < NX; j++) x[u][j] = gr_ldx<WFMT, WIDE>(xb, xl, ui(u), j);
     }
     if constexpr (NORM) {
-        const GrPtr nb = gr_base(a.norm_w, (uint64_t)u0 * (2 * gr_uk(WFMT)));
+        const GblPtr nb = gbl_base(a.norm_w, (uint64_t)u0 * (2 * gr_uk(WFMT)));
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
@@ -461,7 +424,7 @@ __global__ __launch_bounds__(64 * NW) void k_gvr(GvrArgs a) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
 #pragma unroll
-        for (int j = 0; j < NX; j++) x[u][j] = gr_order<WFMT>(x[u][j]);
+        for (int j = 0; j < NX; j++) x[u][j] = WFMT == GEMV_W_INT4 ? int4_order(x[u][j]) : x[u][j];
         if constexpr (!TAIL) gr_bias<WFMT, NX>(x[u], cb[u]);
     }
 
@@ -542,7 +505,7 @@ __global__ __launch_bounds__(64 * GS_WAVES) void k_gvs(GvrArgs a) {
     /* rows past M repeat the last one, their outputs are dropped */
     const uint32_t xl = (uint32_t)min(WIDE ? r : (r & 7), a.M - 1) * (uint32_t)a.ldx * 2u +
                         gr_klane<WFMT, WIDE>(q, hi);
-    const GrPtr xb = gr_base(a.x, (uint64_t)u0 * (2 * gr_uk(WFMT)));
+    const GblPtr xb = gbl_base(a.x, (uint64_t)u0 * (2 * gr_uk(WFMT)));
 
     /* chunk t of the current round (past the slice: its last unit again) */
     GvrTile<WFMT, WIDE> tl[NT];
@@ -568,7 +531,7 @@ __global__ __launch_bounds__(64 * GS_WAVES) void k_gvs(GvrArgs a) {
             s2p_u32x4 x[NX];
             s2p_f32x4 cb[NX];
 #pragma unroll
-            for (int j = 0; j < NX; j++) x[j] = gr_order<WFMT>(c.x[i][j]);
+            for (int j = 0; j < NX; j++) x[j] = WFMT == GEMV_W_INT4 ? int4_order(c.x[i][j]) : c.x[i][j];
             gr_bias<WFMT, NX>(x, cb);
 #pragma unroll
             for (int j = 0; j < NT; j++) gr_mul<WFMT, WIDE>(c.b[i][j], x, cb, hi, acc[j]);

@@ -1,11 +1,10 @@
 /* s2pro MI355X — quantised linear layers (reference src/sched/gemm.c) and
  * the raw GEMV entry points of include/s2pro/gemm.h.
  *
- * One process-wide context (reference gemm.c:42-73) owns the split-K partial
- * buffer and the per-row-block arrival counters of the GEMV engine; GEMVs
- * issued on one stream reuse them in order.  The split count of each call is
- * chosen so that about 4 workgroups per CU stream the weights while each
- * split covers at least 8 groups of 32 k. */
+ * One process-wide context (reference gemm.c:42-73) owns the scratch of the
+ * GEMV / GEMM kernels (packed activations, K-split partials, the split-K
+ * engine's per-row-block arrival counters); calls issued on one stream reuse it
+ * in order. */
 #include <pthread.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -121,7 +120,8 @@ s2p_status s2p_gemm_bf16(const void* x, const void* w, void* y, int M, int N, in
     if (!g.inited) return S2P_ERR_STATE;
     hipError_t e = hipSuccess;
     if (K % 128 == 0) {
-        /* whole-K engine, in row chunks whose activations fit in LDS */
+        /* up to 128 rows a launch; fewer where no engine takes them (few rows of a
+         * K whose activations do not fit in LDS, no room for the packed ones) */
         int mc = M < GEMV_MAX_M ? M : GEMV_MAX_M;
         for (int m0 = 0; m0 < M;) {
             const int rows = M - m0 < mc ? M - m0 : mc;

@@ -28,6 +28,7 @@
 #include <stdint.h>
 
 #include "common.h"
+#include "prims_internal.h"
 #include "s2pro/s2p_fmath.h"
 #include "s2pro/slowar_kernels.h"
 
@@ -215,15 +216,6 @@ __global__ __launch_bounds__(KV8_TILE) void k_attention8_split(
         part[pi * 2 + 1] = l;
     }
 }
-
-extern "C" hipError_t s2p_attn_combine_launch(const float* part, uint16_t* out, int rows, int qh,
-                                              int nsplit, hipStream_t st);
-
-extern "C" hipError_t s2p_attn_dec_launch(const uint16_t* q, const void* const* kcs,
-                                          const void* const* vcs, const uint16_t* const* kss,
-                                          const uint16_t* const* vss, uint16_t* out, int rows,
-                                          int kv_heads, const int32_t* pos, int max_seq,
-                                          int max_len, float* part, int bw, hipStream_t st);
 
 extern "C" hipError_t s2pk_kv_append8(const s2p_bf16* k, const s2p_bf16* v, int8_t* k_cache,
                                       int8_t* v_cache, void* k_scale, void* v_scale, int rows,

@@ -102,8 +102,9 @@ hipError_t s2p_attn_plan_launch(const void* q, void* out, const S2pRowPlan* plan
                                 const S2pAttnSeg* segs, int n_seg, int rows, int layer,
                                 int max_span, float* part, hipStream_t st);
 /* The same, fused with qk-norm + RoPE + KV append (q is the scratch the q
- * rows are written to; no segment has more than max_nrows <= 8 rows) and, with counters ([n_seg * 8], zero between calls),
- * with the split merge done by the last split of each block. */
+ * rows are written to; no segment has more than max_nrows <= 8 rows) and, with
+ * counters ([n_seg * 8], zero between calls), with the split merge done by the
+ * last split of each block. */
 /* qn_w = kn_w = NULL: RoPE without qk-norm (a model without qk-norm) */
 /* Tree attention over bf16 caches (csrc/attention.hip): segs [n_seg] hold
  * one segment a session of max_nrows <= 32 rows; q holds the roped rows
@@ -119,6 +120,17 @@ hipError_t s2p_attn_plan_fused_launch(void* q, void* out, const S2pRowPlan* plan
                                       const void* qn_w, const void* kn_w, const float* rope_tab,
                                       float eps, unsigned* counters, hipStream_t st);
 int64_t    s2p_attn_plan_part_floats(int rows, int max_span);
+
+/* Lockstep decode (csrc/attn_decode.hip): one row a session over its own cache,
+ * bw 16 (bf16), 8 or 4; 4 kv_heads query heads; kss / vss: f16 scales (bw 8, 4);
+ * part: ceil(max_len / 128) splits a (row, head), 130 floats each. */
+hipError_t s2p_attn_dec_launch(const uint16_t* q, const void* const* kcs, const void* const* vcs,
+                               const uint16_t* const* kss, const uint16_t* const* vss,
+                               uint16_t* out, int rows, int kv_heads, const int32_t* pos,
+                               int max_seq, int max_len, float* part, int bw, hipStream_t st);
+/* the splits' partials of every (row, head), merged in split order */
+hipError_t s2p_attn_combine_launch(const float* part, uint16_t* out, int rows, int qh, int nsplit,
+                                   hipStream_t st);
 
 /* The verify plan over INT8 / INT4 (bw 8 / 4) session caches (kv8.hip): codes
  * plan.kv[s] [layers][16][max_seq][bw == 8 ? 128 : 64] (K heads, then V) and
