@@ -372,8 +372,8 @@ static int ad_rounds(int pairs, int units, bool bf16) {
     }
     int best = units;
     int64_t least = INT64_MAX;
-    for (int k = 1; k <= most || k == 1; k++) {
-        const int ups = (units + k - 1) / k, n = (units + ups - 1) / ups;
+    for (int n = 1; n <= most || n == 1;) { /* the split counts that whole rounds give */
+        const int ups = (units + n - 1) / n;
         int64_t per_cu = ((int64_t)n * pairs + cus - 1) / cus;
         if (per_cu < 2) per_cu = 2;
         const int64_t cost = per_cu * (20 * (int64_t)ups + 10) + (n > 1 ? 20 + n : 0);
@@ -382,6 +382,8 @@ static int ad_rounds(int pairs, int units, bool bf16) {
             best = ups;
         }
         if (ups == 1) break;
+        const int u = (units - 1) / n; /* the most rounds a split of the next count */
+        n = (units + u - 1) / u;
     }
     return best;
 }
